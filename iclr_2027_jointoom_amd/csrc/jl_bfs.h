@@ -1,17 +1,17 @@
 // jl_bfs.h - wavefront-level bit-parallel BFS over one map.
 //
-// One 64-lane wavefront runs one BFS.  Lane l owns map rows x = l + 64*r
-// (r < R, so W <= 64*R); a row is held as HW 64-bit masks over its H
-// columns.  A level expands the frontier with shifts inside the row
-// (y +- 1, carrying across words) and with the frontier rows of the lanes
-// above/below (x +- 1, via DPP whole-wavefront shifts by one lane, and
-// readlane across the 64-row groups), masks with free & ~visited, and
-// stops when no lane found a new cell.  Newly reached cells get their level
-// written into an LDS distance array; every other access is a register op,
-// so a level costs O(R*HW) VALU work instead of one thread per frontier
-// node with two workgroup barriers (energy_map.cu:174-245,
-// mapf_gpt_cuda.cu:255-318).  BFS distances are unique, so the field
-// equals the reference's level-synchronous queue BFS.
+// A map row is held as bit masks over its columns.  A level expands the
+// frontier with shifts inside the row (y +- 1, carrying across words) and
+// with the frontier rows above and below (x +- 1: another register or a DPP
+// whole-wavefront shift by one lane), masks with the free cells not reached
+// yet, and stops when no lane found a new cell.  Every access but the final
+// stores is a register op, so a level costs a few VALU instructions per word
+// instead of one thread per frontier node with two workgroup barriers
+// (energy_map.cu:174-245, mapf_gpt_cuda.cu:255-318).  BFS distances are
+// unique, so the field equals the reference's level-synchronous queue BFS.
+//
+// wave_bfs, wave_bfs_batched, wave_bfs_levels: rows of 64-bit words, row x =
+// lane + 64 r.  search_rows: maps of any size, R consecutive rows per lane.
 #pragma once
 
 #include "jl_common.h"
@@ -105,10 +105,9 @@ __device__ __forceinline__ void load_free_rows(const uint32_t* __restrict__ env_
 // even when it is an obstacle, as the energy BFS does) and writes
 // dist[x*H+y] = level for every reached cell except the start, for levels
 // 1..cap.  dist must already hold the "unreached" value and the start cell
-// its 0.  Returns the sum over levels of max(0, level_size - 4096) when
-// kCountOverflow (the nodes the reference's 4096-entry frontier would drop).
-template <int H, int R, typename T, bool kCountOverflow>
-__device__ int wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int gy, int cap,
+// its 0.
+template <int H, int R, typename T>
+__device__ void wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int gy, int cap,
                         T* dist) {
     constexpr int HW = RowWords<H>::HW;
     const int lane = threadIdx.x & (kWave - 1);
@@ -137,7 +136,6 @@ __device__ int wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int gy
             }
         }
     }
-    int overflow = 0;
     for (int level = 1; level <= cap; ++level) {
         uint64_t nf[R][HW];
         bool any_new = false;
@@ -167,7 +165,6 @@ __device__ int wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int gy
             }
         }
         if (!__any(any_new)) break;
-        int local = 0;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int x = lane + kWave * r;
@@ -175,7 +172,6 @@ __device__ int wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int gy
             for (int k = 0; k < HW; ++k) {
                 front[r][k] = nf[r][k];
                 uint64_t m = nf[r][k];
-                if (kCountOverflow) local += __popcll(m);
                 // two new cells per pass, the lowest and the highest (the same
                 // cell twice when one is left)
                 T* row_dist = dist + x * H + k * 64;
@@ -188,19 +184,11 @@ __device__ int wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int gy
                 }
             }
         }
-        // a level of more than kMaxFrontier = 64 * 64 cells has a lane with
-        // more than 64 of them, so the sum is only needed then
-        if (kCountOverflow && __any(local > kMaxFrontier / kWave)) {
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) local += __shfl_xor(local, off, kWave);
-            if (local > kMaxFrontier) overflow += local - kMaxFrontier;
-        }
     }
-    return overflow;
 }
 
-// wave_bfs for one row per lane (R = 1) without the frontier overflow count
-// and without a level cap, in batches of 16 levels: the levels of a batch
+// wave_bfs for one row per lane (R = 1) without a level cap, in batches of 16
+// levels: the levels of a batch
 // are unrolled into straight-line code (expansion, then the new cells ORed
 // into the batch mask and into the planes of the level's 4 low bits, chosen
 // at compile time), and only after the batch are its cells' distances
@@ -345,155 +333,6 @@ __device__ void wave_bfs_levels(uint64_t fr, int gx, int gy, uint64_t& vis, uint
     lowp[0] = vis & odd_cols;
 }
 
-// Free-cell masks of map row x (0 for x >= W), for the group BFS.
-template <int H>
-__device__ __forceinline__ void load_free_row(const uint32_t* __restrict__ env_bits, int W, int x,
-                                              uint64_t (&fr)[RowWords<H>::HW]) {
-    constexpr int HW = RowWords<H>::HW;
-#pragma unroll
-    for (int k = 0; k < HW; ++k) {
-        uint64_t v = 0;
-        if (x < W) {
-            const uint32_t* row = env_bits + (size_t)x * (H / 32);
-            if (H == 32) {
-                v = (uint64_t)(~row[0]) & 0xFFFFFFFFull;
-            } else {
-                const uint64_t hi = 2 * k + 1 < H / 32 ? row[2 * k + 1] : 0xFFFFFFFFu;  // half a word (H % 64 == 32)
-                v = ~((uint64_t)row[2 * k] | (hi << 32));
-            }
-            if (k == HW - 1) v &= RowWords<H>::kLastMask;
-        }
-        fr[k] = v;
-    }
-}
-
-// LDS words the group BFS needs besides the distance array (64-bit words):
-// the boundary rows [2 parities][R wavefronts][top, bottom][HW], then the
-// per-wavefront flags [2][R] and counts [R] (one word each).
-template <int H, int R>
-__host__ __device__ constexpr int group_bfs_words() {
-    return 2 * R * 2 * RowWords<H>::HW + 2 * R + R;
-}
-
-// wave_bfs over a workgroup of R wavefronts (R > 1; every wavefront of the
-// workgroup calls it with the same arguments and all lanes active):
-// wavefront w owns map rows x = 64 w + lane, each held as HW 64-bit masks
-// (fr: this lane's row).  A level is wave_bfs's on the wavefront's rows; the
-// frontier rows at a wavefront boundary (64 w - 1 and 64 w + 64) travel
-// through LDS, written at the end of the level before and read by this one,
-// in slots alternating with the level's parity, with one workgroup barrier
-// per level.  Each wavefront publishes with its boundary rows whether it
-// found a new cell, and every wavefront stops at the first level at which
-// none did.  The frontier overflow count needs the level's total over the
-// workgroup, taken (with a second barrier) only at levels where some row
-// holds more than kMaxFrontier / (64 R) new cells, as a level of more than
-// kMaxFrontier cells must have one.  Same result as wave_bfs with R rows per
-// lane.
-template <int H, int R, typename T, bool kCountOverflow>
-__device__ int group_bfs(const uint64_t (&fr)[RowWords<H>::HW], int gx, int gy, int cap, T* dist,
-                         uint64_t* s_words) {
-    constexpr int HW = RowWords<H>::HW;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    const int x = wave * kWave + lane;
-    uint64_t* s_edge = s_words;                                      // [2][R][2][HW]
-    int* s_flag = reinterpret_cast<int*>(s_words + 2 * R * 2 * HW);  // [2][R], one word apart
-    int* s_count = s_flag + 2 * 2 * R;                               // [R]
-    uint64_t front[HW], vis[HW];
-#pragma unroll
-    for (int k = 0; k < HW; ++k) {
-        front[k] = 0;
-        vis[k] = 0;
-    }
-    if (x == gx) {
-#pragma unroll
-        for (int k = 0; k < HW; ++k) {
-            if (k == (gy >> 6)) {
-                front[k] = 1ull << (gy & 63);
-                vis[k] = front[k];
-            }
-        }
-    }
-    // boundary rows of slot `slot`: lane 0 stores the top row, lane 63 the bottom one
-    auto publish = [&](int slot, const uint64_t (&f)[HW], int flag) {
-        uint64_t* e = s_edge + (size_t)((slot * R + wave) * 2) * HW;
-        if (lane == 0) {
-#pragma unroll
-            for (int k = 0; k < HW; ++k) e[k] = f[k];
-            s_flag[2 * (slot * R + wave)] = flag;
-        }
-        if (lane == kWave - 1) {
-#pragma unroll
-            for (int k = 0; k < HW; ++k) e[HW + k] = f[k];
-        }
-    };
-    publish(1, front, 1);  // level 1 reads the start's rows from slot 1
-    __syncthreads();
-    constexpr int kBigRow = kMaxFrontier / (kWave * R);
-    int overflow = 0;
-    for (int level = 1; level <= cap; ++level) {
-        const int rd = level & 1, wr = rd ^ 1;
-        uint64_t nf[HW];
-        bool any_new = false;
-        int local = 0;
-#pragma unroll
-        for (int k = 0; k < HW; ++k) {
-            uint64_t up = from_lane_below(front[k]);
-            uint64_t down = from_lane_above(front[k]);
-            if (lane == 0 && wave > 0) up = s_edge[(size_t)((rd * R + wave - 1) * 2 + 1) * HW + k];
-            if (lane == kWave - 1 && wave + 1 < R) down = s_edge[(size_t)((rd * R + wave + 1) * 2) * HW + k];
-            uint64_t left = front[k] << 1;
-            uint64_t right = front[k] >> 1;
-            if (k > 0) left |= front[k - 1] >> 63;
-            if (k + 1 < HW) right |= front[k + 1] << 63;
-            const uint64_t n = (left | right | up | down) & fr[k] & ~vis[k];
-            nf[k] = n;
-            any_new |= (n != 0);
-            if (kCountOverflow) local += __popcll(n);
-        }
-        const bool wave_new = __any(any_new);
-        const bool big = kCountOverflow && __any(local > kBigRow);
-        publish(wr, nf, (wave_new ? 1 : 0) | (big ? 2 : 0));
-#pragma unroll
-        for (int k = 0; k < HW; ++k) {
-            vis[k] |= nf[k];
-            front[k] = nf[k];
-            uint64_t m = nf[k];
-            T* row_dist = dist + x * H + k * 64;
-            while (m) {
-                const int lo = __ffsll((unsigned long long)m) - 1;
-                const int hi = 63 - __clzll((long long)m);
-                row_dist[lo] = (T)level;
-                row_dist[hi] = (T)level;
-                m &= ~((1ull << lo) | (1ull << hi));
-            }
-        }
-        __syncthreads();
-        int flags = 0;
-#pragma unroll
-        for (int w = 0; w < R; ++w) flags |= s_flag[2 * (wr * R + w)];
-        flags = __builtin_amdgcn_readfirstlane(flags);
-        if (kCountOverflow && (flags & 2)) {
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) local += __shfl_xor(local, off, kWave);
-            if (lane == 0) s_count[wave] = local;
-            __syncthreads();
-            int total = 0;
-#pragma unroll
-            for (int w = 0; w < R; ++w) total += s_count[w];
-            total = __builtin_amdgcn_readfirstlane(total);
-            if (total > kMaxFrontier) overflow += total - kMaxFrontier;
-            __syncthreads();  // s_count is rewritten at a later level
-        }
-        if (!(flags & 1)) break;
-    }
-    return overflow;
-}
-
-// Bit-planes of BFS levels: a reached cell's level (below 2^kLevelPlanes)
-// is held bit-sliced, plane b holding bit b of the levels of a row's cells.
-constexpr int kLevelPlanes = 16;
-
 // 8x8 bit-matrix transpose: bit c of byte b moves to bit b of byte c.
 __device__ __forceinline__ uint64_t transpose8x8(uint64_t x) {
     uint64_t t = (x ^ (x >> 7)) & 0x00AA00AA00AA00AAull;
@@ -505,135 +344,368 @@ __device__ __forceinline__ uint64_t transpose8x8(uint64_t x) {
     return x;
 }
 
-// group_bfs keeping each reached cell's level in registers instead of an LDS
-// distance array: at level L the new frontier is ORed into the planes of
-// L's set bits, so no per-cell write happens during the search.  On return
-// vis holds the reached cells of this lane's row (the start included, at
-// level 0) and `top` the last level that reached a cell.  s_words as for
-// group_bfs.
-template <int H, int R, bool kCountOverflow>
-__device__ int group_bfs_planes(const uint64_t (&fr)[RowWords<H>::HW], int gx, int gy,
-                                uint64_t (&vis)[RowWords<H>::HW],
-                                uint64_t (&pl)[kLevelPlanes][RowWords<H>::HW], int& top, uint64_t* s_words) {
-    constexpr int HW = RowWords<H>::HW;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    const int x = wave * kWave + lane;
-    uint64_t* s_edge = s_words;
-    int* s_flag = reinterpret_cast<int*>(s_words + 2 * R * 2 * HW);
-    int* s_count = s_flag + 2 * 2 * R;
-    uint64_t front[HW], avail[HW];  // avail: free cells not reached yet
+// ---------------------------------------------------------------------------
+// Row search: one field on a map whose rows do not fit one 64-bit word per
+// lane.  A lane holds R consecutive map rows (x = row0 + R * lane + r) as
+// H / 32 words each, so a row's x +- 1 neighbours are another register of
+// the lane or, at the ends of its block, one DPP lane move: no word of the
+// search leaves the registers.  A level costs six VALU instructions per word
+// (two funnel shifts, two ORs, two three-input bit operations).
+// Levels are held bit-sliced: bit 0 is the parity of the Manhattan offset from
+// the goal, as in wave_bfs_levels; a cell's other bits follow the search
+// until the cell is reached, which freezes them: whenever a level's number
+// changes a bit, that bit's plane is flipped at every cell still free (bit 1
+// after each odd level, bit 2 after every fourth, ...).  Bits 1-3 and kHigh
+// more are planes in registers; the planes of higher bits, flipped rarely
+// (bit k once in 2^k levels), lie in the memory of the field being searched,
+// which the caller writes last (TallPlanes).
+//
+// Split (kSplit): maps of more rows than one wavefront's 64 R are split over
+// the wavefronts of a workgroup.  Neighbouring wavefronts overlap: each also
+// searches the kGhost lanes of rows beyond its own on either side, which stay
+// right in its own rows for kGhost * R = 8 levels; after every 8 levels the
+// owners' rows replace the overlap through LDS.  One barrier in 8 levels,
+// against one per level with the boundary rows alone (256 x 256: five
+// wavefronts instead of four, but 8 times fewer barriers and LDS round trips).
+// A wavefront none of whose rows, overlap included, holds a frontier cell
+// leaves those 8 levels out.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t word_from_below(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xF, 0xF, true);
+}
+
+__device__ __forceinline__ uint32_t word_from_above(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xF, 0xF, true);
+}
+
+constexpr int kSplitLevels = 8;  // levels between two exchanges of a split search
+
+template <int H, int R>
+struct SearchShape {
+    static constexpr int HW = H / 32;              // words per row
+    static constexpr int N = R * HW;               // words per lane
+    static constexpr int kGhost = kSplitLevels / R;  // overlapping lanes on each side of a split
+    static constexpr int kStep = (kWave - 2 * kGhost) * R;  // rows from one wavefront of a split to the next
+    static constexpr int kMaxWaves = (256 - kWave * R + kStep - 1) / kStep + 1;
+    static_assert(kSplitLevels % R == 0 && H % 32 == 0, "row search shape");
+};
+
+// Wavefronts of a split search of W rows (tile rows past W included).
+template <int H, int R>
+__host__ __device__ constexpr int split_waves(int W) {
+    const int rows = (W + 7) / 8 * 8;
+    return rows <= kWave * R ? 1
+                             : (rows - kWave * R + SearchShape<H, R>::kStep - 1) / SearchShape<H, R>::kStep + 1;
+}
+
+// Bits of the levels of a search over `cells` cells (levels stay below it).
+__host__ __device__ constexpr int level_bits(int cells) {
+    int b = 0;
+    while ((1 << b) < cells) ++b;
+    return b;
+}
+
+// LDS of the searches of a workgroup of kWaves wavefronts.
+template <int H, int R, bool kSplit, bool kCount, int kWaves>
+struct SearchLds {
+    using S = SearchShape<H, R>;
+    uint2 edge[kSplit ? 2 : 1][kSplit ? kWaves : 1][2][kSplit ? S::N : 1][S::kGhost];  // a split's frontier and free rows
+    uint32_t before[kCount ? kWaves : 1][kCount ? S::N * kWave : 1];                   // free cells before a batch
+    uint32_t flag[2][kWaves];                                                          // count << 1 | frontier left
+    uint32_t count[16];
+    uint32_t cell[8];
+};
+
+// One wavefront's part of a search's result.
+template <int H, int R, int kHigh>
+struct SearchPlanes {
+    static constexpr int N = SearchShape<H, R>::N;
+    uint32_t avail[N];           // free cells not reached
+    uint32_t low[3][N];          // level bits 1..3
+    uint32_t high[kHigh][N];     // level bits 4 .. 3 + kHigh
+    int tall;                    // planes of the bits above in use (TallPlanes)
+    int batches;                 // of 16 levels searched: every level is at most 16 * batches
+};
+
+// One lane's words.
+template <int H, int R>
+using LaneWords = uint32_t[SearchShape<H, R>::N];
+
+// One level: the frontier's free neighbours become the frontier.
+template <int H, int R>
+__device__ __forceinline__ void expand_rows(LaneWords<H, R>& f, LaneWords<H, R>& av) {
+    constexpr int HW = SearchShape<H, R>::HW, N = SearchShape<H, R>::N;
+    uint32_t n[N];
 #pragma unroll
-    for (int k = 0; k < HW; ++k) {
-        front[k] = 0;
-        avail[k] = fr[k];
-#pragma unroll
-        for (int b = 0; b < kLevelPlanes; ++b) pl[b][k] = 0;
+    for (int i = 0; i < N; ++i) {
+        const int r = i / HW, k = i % HW;
+        const uint32_t up = r > 0 ? f[r > 0 ? i - HW : 0] : word_from_below(f[(R - 1) * HW + k]);
+        const uint32_t down = r + 1 < R ? f[r + 1 < R ? i + HW : 0] : word_from_above(f[k]);
+        const uint32_t left = k > 0 ? __builtin_amdgcn_alignbit(f[i], f[k > 0 ? i - 1 : 0], 31) : f[i] << 1;
+        const uint32_t right = k + 1 < HW ? __builtin_amdgcn_alignbit(f[k + 1 < HW ? i + 1 : 0], f[i], 1) : f[i] >> 1;
+        const uint32_t a = up | right, b = down | left;
+        n[i] = (uint32_t)__builtin_amdgcn_bitop3_b32(a, b, av[i], 0xA8);   // (a | b) & av
+        av[i] = (uint32_t)__builtin_amdgcn_bitop3_b32(a, b, av[i], 0x02);  // av & ~(a | b)
     }
-    if (x == gx) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) f[i] = n[i];
+    // levels are not interleaved: a level's words are independent enough, and
+    // two levels' worth of them would not fit the registers
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// p ^= a for every word.
+template <int N>
+__device__ __forceinline__ void flip_rows(uint32_t (&p)[N], const uint32_t (&a)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] ^= a[i];
+}
+
+template <int N>
+__device__ __forceinline__ bool any_row(const uint32_t (&v)[N]) {
+    uint32_t o = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) o |= v[i];
+    return o != 0;
+}
+
+// Sum over the wavefront's lanes, wavefront-uniform (DPP steps that leave it in lane 63).
+__device__ __forceinline__ int wave_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
+    v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
+    v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);  // row_half_mirror
+    v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false);  // row_mirror
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast31 into rows 2 and 3
+    return __builtin_amdgcn_readlane(v, kWave - 1);
+}
+
+// Free-cell words of a lane's rows, from map row x0 on (0 for rows past W).
+template <int H, int R>
+__device__ __forceinline__ void load_search_rows(const uint32_t* __restrict__ env_bits, int W, int x0,
+                                                 LaneWords<H, R>& fr) {
+    constexpr int HW = SearchShape<H, R>::HW;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int x = x0 + r;
+        const uint32_t* row = env_bits + (size_t)(x < W ? x : 0) * HW;
 #pragma unroll
         for (int k = 0; k < HW; ++k) {
-            if (k == (gy >> 6)) {
-                front[k] = 1ull << (gy & 63);
-                avail[k] &= ~front[k];
-            }
+            const uint32_t w = row[k];
+            fr[r * HW + k] = x < W ? ~w : 0u;
         }
     }
+}
+
+// Lanes of this wavefront whose rows are its own (the others overlap a
+// neighbour's, whose copy counts).
+template <int H, int R, bool kSplit>
+__device__ __forceinline__ bool own_lane(int lane, int wave, int waves) {
+    if (!kSplit) return true;
+    constexpr int G = SearchShape<H, R>::kGhost;
+    return (lane >= G || wave == 0) && (lane < kWave - G || wave + 1 == waves);
+}
+
+// No planes past the register ones (searches capped below 2^(4 + kHigh) levels).
+struct NoTallPlanes {
+    template <int N>
+    __device__ __forceinline__ void flip(int, bool, const uint32_t (&)[N]) const {}
+};
+
+// The search from (gx, gy) (inside the map; reached whether free or not) over
+// the free rows in P.avail.  kCap: levels from 16 * kCap on stay unreached
+// (0: no cap).  Returns, when kCount, the sum over levels of max(0, cells -
+// kMaxFrontier).  Every lane of the wavefront (kSplit: of the workgroup)
+// calls it with the same goal, and with the first of its map rows in x0.
+template <int H, int R, bool kSplit, int kHigh, int kCap, bool kCount, typename Lds, typename Tall>
+__device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx, int gy, int x0, int lane, int wave, int waves,
+                                           Lds& s, const Tall& tall) {
+    using S = SearchShape<H, R>;
+    constexpr int HW = S::HW, N = S::N, G = S::kGhost;
+    const bool own = own_lane<H, R, kSplit>(lane, wave, waves);
+    // the free cells before a batch, read back only where its levels are
+    // counted (volatile: kept in LDS, not forwarded through registers)
+    volatile uint32_t* before = s.before[kCount ? wave : 0] + lane;
+    uint32_t f[N];
+    P.tall = 0;
 #pragma unroll
-    for (int k = 0; k < HW; ++k) vis[k] = front[k];  // the start, obstacle or not
-    auto publish = [&](int slot, const uint64_t (&f)[HW], int flag) {
-        uint64_t* e = s_edge + (size_t)((slot * R + wave) * 2) * HW;
-        if (lane == 0) {
+    for (int i = 0; i < N; ++i) {
+        f[i] = (x0 + i / HW == gx && i % HW == (gy >> 5)) ? 1u << (gy & 31) : 0u;
+        P.avail[i] &= ~f[i];
+        P.low[0][i] = P.low[1][i] = P.low[2][i] = 0;
 #pragma unroll
-            for (int k = 0; k < HW; ++k) e[k] = f[k];
-            s_flag[2 * (slot * R + wave)] = flag;
+        for (int p = 0; p < kHigh; ++p) P.high[p][i] = 0;
+    }
+    auto free_cells = [&]() -> int {
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) c += __popc(P.avail[i]);
+        return c;
+    };
+    int slot = 0, cells = kCount ? free_cells() : 0;
+    bool big = false;  // kCount: 8 levels of the batch reached more than kMaxFrontier cells
+    // After kSplitLevels levels: whether any cell is left to expand; sets
+    // big.  kSplit: the overlap is taken from its owners.
+    auto meet = [&]() -> bool {
+        const bool left = any_row(f);
+        int reached = 0;
+        if (kCount) {
+            const int now = free_cells();
+            reached = cells - now;
+            cells = now;
         }
-        if (lane == kWave - 1) {
+        if constexpr (!kSplit) {
+            // more than kMaxFrontier cells need a lane with more than its share
+            if (kCount && __any(reached > kMaxFrontier / kWave)) big |= wave_sum(reached) > kMaxFrontier;
+            return __any(left) != 0;
+        } else {
+            const bool lo = lane >= G && lane < 2 * G, hi = lane >= kWave - 2 * G && lane < kWave - G;
+            if (lo || hi) {
+                uint2* out = &s.edge[slot][wave][hi ? 1 : 0][0][hi ? lane - (kWave - 2 * G) : lane - G];
 #pragma unroll
-            for (int k = 0; k < HW; ++k) e[HW + k] = f[k];
+                for (int i = 0; i < N; ++i) out[i * G] = make_uint2(f[i], P.avail[i]);
+            }
+            const bool mine = __any(left && own) != 0;
+            const int sum = kCount ? wave_sum(own ? reached : 0) : 0;
+            if (lane == 0) s.flag[slot][wave] = (uint32_t)sum << 1 | (mine ? 1u : 0u);
+            lds_barrier();
+            const uint32_t all = s.flag[slot][lane < waves ? lane : 0];
+            const bool from_lo = lane < G && wave > 0, from_hi = lane >= kWave - G && wave + 1 < waves;
+            if (from_lo || from_hi) {
+                const uint2* in = from_lo ? &s.edge[slot][wave - 1][1][0][lane]
+                                          : &s.edge[slot][wave + 1][0][0][lane - (kWave - G)];
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    const uint2 v = in[i * G];
+                    f[i] = v.x;
+                    P.avail[i] = v.y;
+                }
+            }
+            slot ^= 1;
+            // (the wavefronts' counts are added up only where one of them
+            // has more than its share)
+            if (kCount && __any((int)(all >> 1) * waves > kMaxFrontier))
+                big |= wave_sum(lane < waves ? (int)(all >> 1) : 0) > kMaxFrontier;
+            return __any(all & 1u) != 0;
         }
     };
-    publish(1, front, 1);
-    __syncthreads();
-    constexpr int kBigRow = kMaxFrontier / (kWave * R);
-    constexpr int kCap = (1 << kLevelPlanes) - 2;  // levels stay below the unreachable value
     int overflow = 0;
-    top = 0;
-    for (int level = 1; level <= kCap; ++level) {
-        const int rd = level & 1, wr = rd ^ 1;
-        uint64_t nf[HW];
-        bool any_new = false;
-        int local = 0;
+    for (int b = 0;; ++b) {
+        // levels 16 b + 1 .. 16 b + 16
+        if (kCount) {
+            big = false;
 #pragma unroll
-        for (int k = 0; k < HW; ++k) {
-            uint64_t up = from_lane_below(front[k]);
-            uint64_t down = from_lane_above(front[k]);
-            if (lane == 0 && wave > 0) up = s_edge[(size_t)((rd * R + wave - 1) * 2 + 1) * HW + k];
-            if (lane == kWave - 1 && wave + 1 < R) down = s_edge[(size_t)((rd * R + wave + 1) * 2) * HW + k];
-            uint64_t left = front[k] << 1;
-            uint64_t right = front[k] >> 1;
-            if (k > 0) left |= front[k - 1] >> 63;
-            if (k + 1 < HW) right |= front[k + 1] << 63;
-            const uint64_t n = level_step(up, down, left, right, avail[k]);
-            nf[k] = n;
-            any_new |= (n != 0);
-            if (kCountOverflow) local += __popcll(n);
+            for (int i = 0; i < N; ++i) before[i * kWave] = P.avail[i];
         }
-        const bool wave_new = __any(any_new);
-        const bool big = kCountOverflow && __any(local > kBigRow);
-        publish(wr, nf, (wave_new ? 1 : 0) | (big ? 2 : 0));
+        if (!kSplit || __any(any_row(f))) {
 #pragma unroll
-        for (int k = 0; k < HW; ++k) front[k] = nf[k];
+            for (int j = 1; j <= kSplitLevels; ++j) {
+                expand_rows<H, R>(f, P.avail);
+                if (j % 2 == 1) flip_rows(P.low[0], P.avail);
+                if (j % 4 == 3) flip_rows(P.low[1], P.avail);
+                if (j == 7) flip_rows(P.low[2], P.avail);
+            }
+        } else {
+            flip_rows(P.low[2], P.avail);  // (the even numbers of flips of bits 1 and 2 cancel)
+        }
+        bool more = meet();
+        if (more) {
+            const bool act = !kSplit || __any(any_row(f));
+            if (act) {
 #pragma unroll
-        for (int b = 0; b < kLevelPlanes; ++b) {
-            if ((level >> b) & 1) {
+                for (int j = 9; j < 2 * kSplitLevels; ++j) {
+                    expand_rows<H, R>(f, P.avail);
+                    if (j % 2 == 1) flip_rows(P.low[0], P.avail);
+                    if (j % 4 == 3) flip_rows(P.low[1], P.avail);
+                }
+            }
+            if (kCap && b + 1 == kCap) break;  // level 16 * kCap stays out
+            // the level's number reaches 16 (b + 1)
+            flip_rows(P.low[2], P.avail);
+            const int hb = __builtin_amdgcn_readfirstlane(b), change = hb ^ (hb + 1);
+            flip_rows(P.high[0], P.avail);
 #pragma unroll
-                for (int k = 0; k < HW; ++k) pl[b][k] |= nf[k];
+            for (int p = 1; p < kHigh; ++p)
+                if ((change >> p) & 1) flip_rows(P.high[p], P.avail);
+            for (int p = 0; change >> (kHigh + p); ++p) {
+                tall.flip(p, p == P.tall, P.avail);
+                if (p == P.tall) P.tall = p + 1;
+            }
+            if (act) expand_rows<H, R>(f, P.avail);
+            more = meet();
+        }
+        if (kCount && big) {
+            // count the cells of each of the batch's levels, told apart by
+            // their four low bits
+            if (kSplit) {
+                lds_barrier();
+                if (threadIdx.x < 16) s.count[threadIdx.x] = 0;
+                lds_barrier();
+            }
+            for (int v = 0; v < 16; ++v) {
+                int c = 0;
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    const int x = x0 + i / HW;
+                    uint32_t m = before[i * kWave] & ~P.avail[i];
+                    m &= ((x + gx + gy + v) & 1) ? 0xAAAAAAAAu : 0x55555555u;
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) m &= ((v >> (p + 1)) & 1) ? P.low[p][i] : ~P.low[p][i];
+                    c += __popc(m);
+                }
+                c = wave_sum(own ? c : 0);
+                if (kSplit) {
+                    if (lane == 0) atomicAdd(&s.count[v], (uint32_t)c);
+                } else if (c > kMaxFrontier) {
+                    overflow += c - kMaxFrontier;
+                }
+            }
+            if (kSplit) {
+                lds_barrier();
+                for (int v = 0; v < 16; ++v) {
+                    const int c = __builtin_amdgcn_readfirstlane((int)s.count[v]);
+                    if (c > kMaxFrontier) overflow += c - kMaxFrontier;
+                }
+                lds_barrier();
             }
         }
-        __syncthreads();
-        int flags = 0;
-#pragma unroll
-        for (int w = 0; w < R; ++w) flags |= s_flag[2 * (wr * R + w)];
-        flags = __builtin_amdgcn_readfirstlane(flags);
-        if (kCountOverflow && (flags & 2)) {
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) local += __shfl_xor(local, off, kWave);
-            if (lane == 0) s_count[wave] = local;
-            __syncthreads();
-            int total = 0;
-#pragma unroll
-            for (int w = 0; w < R; ++w) total += s_count[w];
-            total = __builtin_amdgcn_readfirstlane(total);
-            if (total > kMaxFrontier) overflow += total - kMaxFrontier;
-            __syncthreads();
-        }
-        if (!(flags & 1)) break;
-        top = level;
+        P.batches = b + 1;
+        if (!more) break;
     }
-#pragma unroll
-    for (int k = 0; k < HW; ++k) vis[k] |= fr[k] & ~avail[k];
     return overflow;
 }
 
-// Level of this lane's cell at column y from the planes (kUnreachable when
-// the cell was not reached).
-template <int H>
-__device__ __forceinline__ uint32_t plane_level(const uint64_t (&vis)[RowWords<H>::HW],
-                                                const uint64_t (&pl)[kLevelPlanes][RowWords<H>::HW], int y) {
-    constexpr int HW = RowWords<H>::HW;
-    uint32_t d = 0;
-    bool reached = false;
+// (a, b) of the rows beside this wavefront's own in a split, from their
+// owners into the overlapping lanes (the owners' first and last rows are what
+// a wavefront's rows border on).  Called by the whole workgroup after a
+// search; the caller lets every wavefront past it before the next search.
+template <int H, int R, typename Lds>
+__device__ __forceinline__ void meet_rows(LaneWords<H, R>& a, LaneWords<H, R>& b, int lane, int wave, int waves, Lds& s) {
+    constexpr int N = SearchShape<H, R>::N, G = SearchShape<H, R>::kGhost;
+    lds_barrier();  // the search's last exchange has been read
+    const bool lo = lane >= G && lane < 2 * G, hi = lane >= kWave - 2 * G && lane < kWave - G;
+    if (lo || hi) {
+        uint2* out = &s.edge[0][wave][hi ? 1 : 0][0][hi ? lane - (kWave - 2 * G) : lane - G];
 #pragma unroll
-    for (int k = 0; k < HW; ++k) {
-        if (k == (y >> 6)) {
-            const int bit = y & 63;
-            reached = (vis[k] >> bit) & 1;
+        for (int i = 0; i < N; ++i) out[i * G] = make_uint2(a[i], b[i]);
+    }
+    lds_barrier();
+    const bool from_lo = lane < G && wave > 0, from_hi = lane >= kWave - G && wave + 1 < waves;
+    if (from_lo || from_hi) {
+        const uint2* in = from_lo ? &s.edge[0][wave - 1][1][0][lane] : &s.edge[0][wave + 1][0][0][lane - (kWave - G)];
 #pragma unroll
-            for (int b = 0; b < kLevelPlanes; ++b) d |= (uint32_t)((pl[b][k] >> bit) & 1) << b;
+        for (int i = 0; i < N; ++i) {
+            const uint2 v = in[i * G];
+            a[i] = v.x;
+            b[i] = v.y;
         }
     }
-    return reached ? d : kUnreachable;
+}
+
+// Bytes q of four words, in a word.
+__device__ __forceinline__ uint32_t gather_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t q) {
+    const uint32_t sel = 0x0C0C0400u + q * 0x0101u;
+    return __builtin_amdgcn_perm(b, a, sel) | __builtin_amdgcn_perm(d, c, sel) << 16;
 }
 
 }  // namespace jl

@@ -43,17 +43,23 @@ __device__ __forceinline__ int wrap_dist2(int dx, int dy) {
 constexpr int kScratchAccum = 0;     // [0..3]
 constexpr int kScratchTicket = 4;
 
-// The builder's tiled copies of the distance fields (cost_tiles) of maps of
-// at most 4096 cells carry each reachable cell's greedy-move mask in bits
-// 12-15: a distance there is below 4095 (at most the number of free cells
-// minus one, and a map with every cell free has a far smaller diameter), so
-// it fits in bits 0-11 and a marked value never equals kUnreachable, which
-// unreachable cells keep.  Readers take the distance as field_distance(v,
-// field_mask(W, H)).  cost_to_go, the API tensor, holds plain distances.
+// The builder's tiled copies of the distance fields (cost_tiles) carry each
+// reachable cell's greedy-move mask in bits 12-15 where every distance of the
+// field fits bits 0-11 and no marked value equals kUnreachable, which
+// unreachable cells keep.  On maps of at most 4096 cells that is every field:
+// a distance there is below 4095 (at most the number of free cells minus
+// one, and a map with every cell free has a far smaller diameter).  On larger
+// maps it is the fields whose agent_info has kInfoMarked set: those whose
+// search ended before level 4095.  Readers take the distance as
+// field_distance(v, mask) with the field's mask.  cost_to_go, the API tensor,
+// holds plain distances.
 constexpr int kMarkedCells = 4096;
+constexpr uint32_t kInfoMarked = 1u << 7;  // agent_info: the field carries marks (maps of more than kMarkedCells)
+constexpr uint32_t kMarkedMask = 0x0FFFu;
 __host__ __device__ inline bool marked_fields(int W, int H) { return W * H <= kMarkedCells; }
-__host__ __device__ inline uint32_t field_mask(int W, int H) {
-    return marked_fields(W, H) ? 0x0FFFu : 0xFFFFu;
+// Distance bits of a field with the given agent_info.
+__host__ __device__ inline uint32_t field_mask(int W, int H, uint32_t info) {
+    return marked_fields(W, H) || (info & kInfoMarked) ? kMarkedMask : 0xFFFFu;
 }
 __device__ __forceinline__ uint32_t field_distance(uint32_t v, uint32_t mask) {
     return v == kUnreachable ? v : (v & mask);

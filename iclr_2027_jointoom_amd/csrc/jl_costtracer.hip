@@ -52,6 +52,7 @@ __device__ __forceinline__ int wave_min(int v) { return wave_reduce<false>(v); }
 // the agent's stream (best reset to -1 so the next observation re-anchors it).
 template <int H>
 __global__ __launch_bounds__(256) void reward_goals_kernel(jl_sim_t s, const uint16_t* __restrict__ tiles,
+                                                           const uint32_t* __restrict__ agent_info,
                                                            int32_t* __restrict__ best,
                                                            const int16_t* __restrict__ targets,
                                                            int length, int32_t* __restrict__ cursor,
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(256) void reward_goals_kernel(jl_sim_t s, const uin
     const int k = cursor[i];
     const int xc = x < W ? x : W - 1, yc = y < H ? y : H - 1;
     const int d = (int)field_distance(tiles[(size_t)i * tiled_cells(W, H) + tile_offset(xc, yc, W)],
-                                      field_mask(W, H));
+                                      field_mask(W, H, marked_fields(W, H) ? 0u : agent_info[i]));
     rewards[i] = d < b0 ? 0.1f : 0.0f;
     int bn = min(b0, d);
     const bool hit = x == gx && y == gy;
@@ -96,13 +97,13 @@ __device__ __forceinline__ void observe_agents(const jl_sim_t& s, const jl_mapfg
                                                int nvalid, int lane) {
     const int W = s.map_w, A = s.n_agents;
     const size_t tcells = tiled_cells(W, H);
-    const uint32_t fmask = field_mask(W, H);
     const int words = W * H / 32;
     // lane k < nvalid fetches agent i0 + k's position, best and refresh flag
     const int il = i0 + (lane < nvalid ? lane : 0);
     const int pxl = s.cur_x[il], pyl = s.cur_y[il];
     const int32_t bestl = best[il];
     const int resetl = b.state_packed[(size_t)il * 8 + 7];
+    const uint32_t infol = marked_fields(W, H) ? 0u : b.agent_info[il];
     // window cells t0 = lane, t1 = lane + 64 (a cell when < 121); t = r*11 + c
     // is (cx + r - 5, cy + c - 5)
     const int t0 = lane, t1 = lane + kWave;
@@ -135,6 +136,7 @@ __device__ __forceinline__ void observe_agents(const jl_sim_t& s, const jl_mapfg
 #pragma unroll
     for (int k = 0; k < kObsPer; ++k) {
         if (k >= nvalid) break;  // wavefront-uniform
+        const uint32_t fmask = field_mask(W, H, (uint32_t)__builtin_amdgcn_readlane((int)infol, k));
         const int d0 = (in0[k] && raw0[k] != kUnreachable) ? (int)(raw0[k] & fmask) : -1;
         const int d1 = (in1[k] && raw1[k] != kUnreachable) ? (int)(raw1[k] & fmask) : -1;
         // largest reachable distance in the window (0 if none)
@@ -250,7 +252,7 @@ int check_pair(const jl_sim_t* s, const jl_mapfgpt_t* b) {
         return JL_ERR_ARG;
     if ((int64_t)s->n_envs * s->n_agents > 0x7FFFFFFF) return JL_ERR_ARG;
     if (!s->cur_x || !s->cur_y || !s->goal_x || !s->goal_y || !s->grid_ocp || !b->cost_tiles ||
-        !b->state_packed)
+        !b->state_packed || (!marked_fields(s->map_w, s->map_h) && !b->agent_info))
         return JL_ERR_ARG;
     return JL_OK;
 }
@@ -270,7 +272,7 @@ extern "C" int jl_costtracer_reward_goals(const jl_sim_t* s, const jl_mapfgpt_t*
     const int n = s->n_envs * s->n_agents;
     JL_DISPATCH_H(s->map_h, {
         hipLaunchKernelGGL((reward_goals_kernel<H>), dim3((n + 255) / 256), dim3(256), 0,
-                           (hipStream_t)stream, *s, b->cost_tiles, best, targets, target_length,
+                           (hipStream_t)stream, *s, b->cost_tiles, b->agent_info, best, targets, target_length,
                            cursor, rewards, reached, n);
     });
     return launch_status();

@@ -31,7 +31,7 @@ __device__ void energy_field(const uint32_t* __restrict__ env_bits, int W, int g
     load_free_rows<H, R>(env_bits, W, fr);
     if (lane == 0) s_dist[gx * H + gy] = 0;
     wave_sync();
-    wave_bfs<H, R, uint8_t, false>(fr, gx, gy, kEnergyCap, s_dist);
+    wave_bfs<H, R, uint8_t>(fr, gx, gy, kEnergyCap, s_dist);
     wave_sync();
     const uint4* src = reinterpret_cast<const uint4*>(s_dist);
     uint4* dst = reinterpret_cast<uint4*>(out);

@@ -3,17 +3,15 @@
 // On maps of at most 4096 cells with at most 1024 agents per env an eager
 // build is one launch of the token kernel, one workgroup per env: its phase 0
 // unpacks the env's agents and refreshes their changed fields (the work of
-// 1a and 1b below), then phases 1 and 2 follow.  Otherwise a build is three
-// launches (two on maps of up to 4096 cells, where 1a and 1b are one kernel):
-//   1a. unpack: one lane per agent, no LDS.  Unpacks the state (raw rows or
-//      resident split arrays), refreshes the goal cache and writes every
-//      agent's info word: the greedy-move mask from the kept tiled field, or a
-//      mark when the reset flag is set.  It also clears `diagnostics`.
-//   1b. bfs: a grid sized to the CUs; each wavefront scans a range of info
-//      words and runs the bit-parallel BFS (jl_bfs.h) for the marked agents
-//      in its own LDS field, stores it in 8x8 tiles (cost_tiles; the API
-//      tensor cost_to_go is filled from them on request) and completes the
-//      info word.
+// 1 below), then phases 1 and 2 follow.  Otherwise a build is two launches:
+//   1. unpack: one lane per agent.  Unpacks the state (raw rows or resident
+//      split arrays), refreshes the goal cache and writes every agent's info
+//      word: the greedy-move mask from the kept tiled field, or, where the
+//      goal changed, what the search of its field yields, which the same
+//      launch runs (jl_bfs.h) and stores in 8x8 tiles (cost_tiles; the API
+//      tensor cost_to_go is filled from them on request).  It also clears
+//      `diagnostics`.  unpack_fields_kernel, or unpack_bfs_kernel on maps of
+//      up to 4096 cells.
 //   2. tokens: one 1024-thread workgroup per env (per 512 egos of a larger
 //      env).  Phase 1
 //      stages the env's agents (position, goal, the six ego-independent
@@ -110,7 +108,6 @@ __device__ __forceinline__ uint4 marked_segment(const uint16_t* f, int W, int x,
 // ---------------------------------------------------------------------------
 // Per-agent steps shared by the launches of a build.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kInfoNeedsBfs = 1u << 6;  // agent_info: field to refresh in pass 1b
 
 __device__ __forceinline__ uint4 state_row(uint32_t env, uint32_t agent, uint32_t px, uint32_t py,
                                            uint32_t gx, uint32_t gy, uint32_t action,
@@ -158,49 +155,39 @@ __device__ __forceinline__ uint4 unpack_agent(const jl_mapfgpt_t& b, int i,
     }
     const uint32_t env = (uint32_t)(i / A);
     const uint32_t agent = (uint32_t)(i - (int)env * A);
+    // every load before the first store (which may alias them): one round trip
     const uint32_t tx = (uint16_t)goal_x[i], ty = (uint16_t)goal_y[i];
+    const uint32_t px = (uint16_t)cur_x[i], py = (uint16_t)cur_y[i];
     const uint32_t goal = tx | (ty << 16);
     const bool changed = *gc != goal;
     if (changed) *gc = goal;
-    const uint4 v = state_row(env, agent, (uint16_t)cur_x[i], (uint16_t)cur_y[i], tx, ty, 0u, changed ? 1u : 0u);
+    const uint4 v = state_row(env, agent, px, py, tx, ty, 0u, changed ? 1u : 0u);
     *st = v;
     b.labels[i] = 0;
     return v;
 }
 
 // Greedy mask of an agent at (px, py) on the map whose field this build
-// keeps, from the tiled copy written by an earlier build.  kMarked (maps of
-// at most kMarkedCells cells): the mark of the agent's own cell, one read;
-// an agent on an unreachable cell (an obstacle, or a component without its
-// goal) and unmarked maps read the cross of five cells (1-3 lines).
-template <int H, bool kMarked>
-__device__ __forceinline__ uint32_t kept_greedy(const jl_mapfgpt_t& b, size_t i, int px, int py) {
+// keeps, from the tiled copy written by an earlier build: the mark of the
+// agent's own cell, one read, where the field carries marks; an agent on an
+// unreachable cell (an obstacle, or a component without its goal) and fields
+// without marks read the cross of five cells (1-3 lines).
+template <int H>
+__device__ __forceinline__ uint32_t kept_greedy(const jl_mapfgpt_t& b, size_t i, int px, int py, bool marked) {
     const int W = b.map_w;
     const uint16_t* f = b.cost_tiles + i * tiled_cells(W, H);
-    if (kMarked) {
-        const uint32_t c = f[tile_offset(px, py, W)];
-        if (c != kUnreachable) return c >> 12;
-    }
+    const uint32_t c = f[tile_offset(px, py, W)];
+    if (marked && c != kUnreachable) return c >> 12;
     return greedy_mask<H>([f, W](int x, int y) { return (uint32_t)f[tile_offset(x, y, W)]; }, px, py, W);
 }
 
-// Refresh of one agent's field (mapf_gpt_cost_to_go_kernel, :181-325) by the
-// calling wavefront (every lane, wavefront-uniform arguments): the
-// bit-parallel BFS (jl_bfs.h) from the goal (gx, gy) over env e's free cells
-// in the wavefront's LDS field s_dist (W * H uint16), then the field in 8x8
-// tiles into cost_tiles (with greedy marks when kMarked), 16-byte stores; the
-// row-major cost_to_go is filled from the tiles on request.  Returns the
-// agent's info bits: the frontier overflow count, or kInfoBadGoal for a goal
-// off the map or on an obstacle (an all-unreachable field, :224-236), and the
-// greedy mask at its position (spx, spy) when that is on the map.
-// The map's tiles of the LDS field s_dist (W * H uint16, with greedy marks
-// when kMarked) into agent agent_index's tiled field, 16-byte row segments
-// first, first + stride, ... (the border ring keeps its unreachable cells).
-template <int H, bool kMarked>
+// The map's tiles of the LDS field s_dist (W * H uint16) with greedy marks
+// into agent agent_index's tiled field, 16-byte row segments first, first +
+// stride, ... (the border ring keeps its unreachable cells).
+template <int H>
 __device__ void store_field_tiles(const jl_mapfgpt_t& b, size_t agent_index, const uint16_t* s_dist,
                                   int first, int stride) {
     const int W = b.map_w;
-    const uint4* lds4 = reinterpret_cast<const uint4*>(s_dist);
     uint4* tout = reinterpret_cast<uint4*>(b.cost_tiles + agent_index * tiled_cells(W, H));
     const int map_tile_rows = (W + 7) / 8;
     for (int c = first; c < map_tile_rows * H; c += stride) {
@@ -209,7 +196,7 @@ __device__ void store_field_tiles(const jl_mapfgpt_t& b, size_t agent_index, con
         const int x = tr * 8 + r, y0 = tc * 8;
         const int dst = (tc + 1) * (int)(strip_cells(W) / 8u) + x + 8;  // 16-byte row of strip tc + 1
         const bool in = x < W;  // rows past the map in the last tile row: unreachable
-        uint4 v = kMarked ? marked_segment<H>(s_dist, W, in ? x : 0, y0) : lds4[((in ? x : 0) * H + y0) >> 3];
+        uint4 v = marked_segment<H>(s_dist, W, in ? x : 0, y0);
         v.x = in ? v.x : 0xFFFFFFFFu;
         v.y = in ? v.y : 0xFFFFFFFFu;
         v.z = in ? v.z : 0xFFFFFFFFu;
@@ -229,8 +216,7 @@ __device__ void store_field_tiles(const jl_mapfgpt_t& b, size_t agent_index, con
 // 8-cell tile-row segments, two 8x8 bit transposes per segment (level bits
 // 0-7, then level bits 8-11 and the four mark bits), stored as 16-byte words
 // (consecutive lanes, consecutive rows of a strip).  Same tiles and info
-// bits as refresh_field<H, 1, true> (no level of such a map can overflow the
-// frontier).  Every lane calls it with wavefront-uniform arguments.
+// bits as refresh_field (no level of such a map can overflow the frontier).  Every lane calls it with wavefront-uniform arguments.
 template <int H>
 __device__ uint32_t refresh_field_levels(const jl_mapfgpt_t& b, size_t agent_index, uint32_t e, int gx, int gy,
                                          int spx, int spy, uint64_t* s_high) {
@@ -310,11 +296,21 @@ __device__ uint32_t refresh_field_levels(const jl_mapfgpt_t& b, size_t agent_ind
     return info;
 }
 
-template <int H, int R, bool kMarked, bool kTiles = true>
+// Refresh of one agent's field on a marked map (mapf_gpt_cost_to_go_kernel,
+// :181-325) by the calling wavefront (every lane, wavefront-uniform
+// arguments): the bit-parallel BFS (jl_bfs.h) from the goal (gx, gy) over env
+// e's free cells in the wavefront's LDS field s_dist (W * H uint16), then
+// (kTiles) the field in 8x8 tiles with greedy marks into cost_tiles, 16-byte
+// stores; the row-major cost_to_go is filled from the tiles on request.
+// Returns the agent's info bits: kInfoBadGoal for a goal off the map or on an
+// obstacle (an all-unreachable field, :224-236), and the greedy mask at its
+// position (spx, spy) when that is on the map.  (No level of a map of at most
+// kMarkedCells cells overflows the frontier.)
+template <int H, int R, bool kTiles = true>
 __device__ uint32_t refresh_field(const jl_mapfgpt_t& b, size_t agent_index, uint32_t e, int gx,
                                   int gy, int spx, int spy, uint16_t* s_dist) {
     constexpr int HW = RowWords<H>::HW;
-    if constexpr (R == 1 && HW == 1 && kMarked && kTiles) {
+    if constexpr (R == 1 && HW == 1 && kTiles) {
         // no LDS field on this path: the caller's s_dist (at least
         // kHighPlaneBytes, marked_wave_lds) holds the high level planes
         return refresh_field_levels<H>(b, agent_index, e, gx, gy, spx, spy, reinterpret_cast<uint64_t*>(s_dist));
@@ -333,227 +329,272 @@ __device__ uint32_t refresh_field(const jl_mapfgpt_t& b, size_t agent_index, uin
     bool ok = e < (uint32_t)b.n_envs && (uint32_t)gx < (uint32_t)W && (uint32_t)gy < (uint32_t)H;
     const uint32_t* env_bits = b.grid_bits + (size_t)(ok ? e : 0) * words;
     if (ok && bit_at(env_bits, gx * H + gy)) ok = false;
-    int overflow = 0;
     if (ok) {
         uint64_t fr[R][HW];
         load_free_rows<H, R>(env_bits, W, fr);
         if (lane == 0) s_dist[gx * H + gy] = 0;
         wave_sync();
-        if (W * H > kMaxFrontier + 1) {
-            overflow = wave_bfs<H, R, uint16_t, true>(fr, gx, gy, 0x7FFFFFFF, s_dist);
-        } else if constexpr (R == 1) {
-            // no level of a map this small can overflow the frontier
+        if constexpr (R == 1) {
             wave_bfs_batched<H, uint16_t>(fr[0], gx, gy, s_dist);
         } else {
-            overflow = wave_bfs<H, R, uint16_t, false>(fr, gx, gy, 0x7FFFFFFF, s_dist);
+            wave_bfs<H, R, uint16_t>(fr, gx, gy, 0x7FFFFFFF, s_dist);
         }
     }
     wave_sync();
-    uint32_t info = ok ? (uint32_t)(overflow < 0xFFFFFF ? overflow : 0xFFFFFF) << kInfoOverflowShift
-                       : kInfoBadGoal;
+    uint32_t info = ok ? 0u : kInfoBadGoal;
     if ((uint32_t)spx < (uint32_t)W && (uint32_t)spy < (uint32_t)H)
         info |= greedy_mask<H>([s_dist](int x, int y) { return (uint32_t)s_dist[x * H + y]; }, spx, spy, W);
     if (kTiles) {
-        store_field_tiles<H, kMarked>(b, agent_index, s_dist, lane, kWave);
+        store_field_tiles<H>(b, agent_index, s_dist, lane, kWave);
         wave_sync();  // the LDS field is rewritten by the next refresh
     }
     return info;
 }
 
-// refresh_field (unmarked fields) by a workgroup of R wavefronts on maps of
-// more than 64 rows, without an LDS distance array: the group BFS with
-// bit-sliced levels (jl_bfs.h, wavefront w on rows 64 w .. 64 w + 63), then
-// every lane turns its row into 8-cell tile-row segments (one 8x8 bit
-// transpose per 8 planes and segment) and stores them into the tiled field.
-// The five cells of the greedy mask at (spx, spy) travel through s_gm.  Every
-// thread calls it with the same arguments.  Same tiles and info bits as
-// refresh_field.
+// Wavefronts per SIMD of the field searches and register planes above level
+// bit 3.  Four (at most 128 registers each) where the map is split, so that
+// the second workgroup of five wavefronts finds room on every SIMD; three
+// (168 registers) where every wavefront is on its own: with 128 the shapes of
+// eight words per lane would spill.
+template <bool kSplit>
+constexpr int field_waves_per_simd() {
+    return kSplit ? 4 : 3;
+}
+template <int N, bool kSplit>
+constexpr int field_high() {
+    return !kSplit || N < 6 ? 3 : (N < 8 ? 2 : 1);
+}
+
+// Level planes of the bits past the register planes of a field under search, kept in the tile
+// rows that the finished field will fill: plane p of word k of map row x is
+// component p & 3 of the 16-byte row x of strip 4 k + 1 + (p >> 2).  Each
+// lane reads and writes its own rows' only.
 template <int H, int R>
-__device__ uint32_t refresh_field_group(const jl_mapfgpt_t& b, size_t agent_index, uint32_t e, int gx, int gy,
-                                        int spx, int spy, uint64_t* s_words, uint32_t* s_gm) {
-    constexpr int HW = RowWords<H>::HW;
-    const int W = b.map_w;
-    const int tid = threadIdx.x;
-    const int x = tid;  // this lane's map row
-    const int words = W * H / 32;
-    const size_t tcells = tiled_cells(W, H);
-    bool ok = e < (uint32_t)b.n_envs && (uint32_t)gx < (uint32_t)W && (uint32_t)gy < (uint32_t)H;
-    const uint32_t* env_bits = b.grid_bits + (size_t)(ok ? e : 0) * words;
-    if (ok && bit_at(env_bits, gx * H + gy)) ok = false;
-    uint64_t vis[HW], pl[kLevelPlanes][HW];
-    int top = 0, overflow = 0;
-#pragma unroll
-    for (int k = 0; k < HW; ++k) {
-        vis[k] = 0;
-#pragma unroll
-        for (int p = 0; p < kLevelPlanes; ++p) pl[p][k] = 0;
+struct TallPlanes {
+    static constexpr int HW = H / 32;
+    uint4* rows;           // the field's tile rows, at this lane's first map row
+    uint32_t strip_words;  // 16-byte rows per strip
+    int valid;             // of this lane's R rows, those it owns on the map
+    __device__ __forceinline__ uint32_t* word(int p, int i) const {
+        return reinterpret_cast<uint32_t*>(rows + (size_t)((i % HW) * 4 + 1 + (p >> 2)) * strip_words + i / HW) + (p & 3);
     }
-    if (ok) {
-        uint64_t fr[HW];
-        load_free_row<H>(env_bits, W, x, fr);
-        if (W * H > kMaxFrontier + 1) {
-            overflow = group_bfs_planes<H, R, true>(fr, gx, gy, vis, pl, top, s_words);
-        } else {
-            overflow = group_bfs_planes<H, R, false>(fr, gx, gy, vis, pl, top, s_words);
-        }
-    }
-    // greedy mask at (spx, spy): the owners of the cell and of its four
-    // neighbours publish their levels (slots: cell, x - 1, x + 1, y - 1, y + 1)
-    const bool on_map = (uint32_t)spx < (uint32_t)W && (uint32_t)spy < (uint32_t)H;
-    if (on_map) {
-        if (x == spx) {
-            s_gm[0] = plane_level<H>(vis, pl, spy);
-            s_gm[3] = spy > 0 ? plane_level<H>(vis, pl, spy - 1) : kUnreachable;
-            s_gm[4] = spy + 1 < H ? plane_level<H>(vis, pl, spy + 1) : kUnreachable;
-        }
-        if (x == spx - 1) s_gm[1] = plane_level<H>(vis, pl, spy);
-        if (x == spx + 1 && x < W) s_gm[2] = plane_level<H>(vis, pl, spy);
-        // neighbours off the map have no owner
-        if (tid == 0 && spx == 0) s_gm[1] = kUnreachable;
-        if (tid == 0 && spx + 1 >= W) s_gm[2] = kUnreachable;
-    }
-    __syncthreads();
-    uint32_t info = ok ? (uint32_t)(overflow < 0xFFFFFF ? overflow : 0xFFFFFF) << kInfoOverflowShift
-                       : kInfoBadGoal;
-    if (on_map) {
-        const uint32_t c0 = s_gm[0];
-        const uint32_t n[4] = {s_gm[1], s_gm[2], s_gm[3], s_gm[4]};
-        uint32_t m = 0;
+    template <int N>
+    __device__ __forceinline__ void flip(int p, bool first, const uint32_t (&a)[N]) const {
 #pragma unroll
-        for (int d = 0; d < 4; ++d)
-            if (n[d] != kUnreachable && c0 > n[d]) m |= 8u >> d;
-        info |= m;
-    }
-    // the map's tiles: this lane's row, 8 cells per segment (the border ring
-    // keeps its unreachable cells; rows past W hold no reached cell)
-    const int nplanes = top == 0 ? 0 : 32 - __clz(top);
-    uint4* tout = reinterpret_cast<uint4*>(b.cost_tiles + agent_index * tcells);
-    const int strip_words = (int)(strip_cells(W) / 8u);
-    if (x < (W + 7) / 8 * 8) {
-#pragma unroll
-        for (int k = 0; k < HW; ++k) {
-            const int groups = (H - k * 64) < 64 ? (H - k * 64) / 8 : 8;
-            for (int jj = 0; jj < groups; ++jj) {
-                const int sh = jj * 8;
-                uint64_t lo = 0, hi = 0;
-#pragma unroll
-                for (int p = 0; p < 8; ++p) lo |= ((pl[p][k] >> sh) & 0xFFull) << (8 * p);
-                lo = transpose8x8(lo);
-                if (nplanes > 8) {
-#pragma unroll
-                    for (int p = 0; p < 8; ++p) hi |= ((pl[8 + p][k] >> sh) & 0xFFull) << (8 * p);
-                    hi = transpose8x8(hi);
-                }
-                const uint32_t reached = (uint32_t)(vis[k] >> sh) & 0xFFu;
-                uint32_t w[4];
-#pragma unroll
-                for (int c = 0; c < 8; c += 2) {
-                    uint32_t d0 = (uint32_t)((lo >> (8 * c)) & 0xFF) | ((uint32_t)((hi >> (8 * c)) & 0xFF) << 8);
-                    uint32_t d1 = (uint32_t)((lo >> (8 * c + 8)) & 0xFF) | ((uint32_t)((hi >> (8 * c + 8)) & 0xFF) << 8);
-                    d0 = ((reached >> c) & 1) ? d0 : kUnreachable;
-                    d1 = ((reached >> (c + 1)) & 1) ? d1 : kUnreachable;
-                    w[c / 2] = d0 | (d1 << 16);
-                }
-                const int strip = k * 8 + jj;  // columns 8 strip .. 8 strip + 7
-                tout[(strip + 1) * strip_words + x + 8] = make_uint4(w[0], w[1], w[2], w[3]);
+        for (int i = 0; i < N; ++i) {
+            if (i / HW < valid) {
+                uint32_t* w = word(p, i);
+                *w = first ? a[i] : *w ^ a[i];
             }
         }
     }
-    __syncthreads();  // s_words and s_gm are rewritten by the next refresh
+};
+
+// Refresh of one agent's field on an unmarked map (mapf_gpt_cost_to_go_kernel,
+// :181-325) by the row search (jl_bfs.h): by the calling wavefront, or
+// (kSplit) by the whole workgroup, each wavefront on its rows from row0 on.
+// Every lane calls it with uniform arguments.  Each lane then turns its rows
+// into the field's 8-cell tile-row segments (two 8x8 bit transposes each),
+// stored as 16-byte words.  The greedy mask at the agent's position (spx,
+// spy) follows from the two low level bits of its cell and the neighbours
+// (refresh_field_levels).  Returns the agent's info bits: the frontier
+// overflow count, or kInfoBadGoal for a goal off the map or on an obstacle
+// (an all-unreachable field, :224-236), and the greedy mask.
+template <int H, int R, bool kSplit, typename Lds>
+__device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, size_t agent_index, uint32_t e, int gx,
+                                                       int gy, int spx, int spy, int wave, int waves, Lds& s) {
+    using S = SearchShape<H, R>;
+    constexpr int HW = S::HW, N = S::N, kFieldHigh = field_high<S::N, kSplit>();
+    const int W = b.map_w;
+    // (the lane is taken afresh for every field: the addresses that follow
+    // from it would otherwise be held, or spilled, across the search)
+    int lane = threadIdx.x & (kWave - 1);
+    asm volatile("" : "+v"(lane));
+    const int row0 = kSplit ? wave * S::kStep : 0;
+    bool ok = e < (uint32_t)b.n_envs && (uint32_t)gx < (uint32_t)W && (uint32_t)gy < (uint32_t)H;
+    const uint32_t* env_bits = b.grid_bits + (size_t)(ok ? e : 0) * (W * H / 32);
+    if (ok && bit_at(env_bits, gx * H + gy)) ok = false;
+    // this lane's rows in the field's tiles (the border ring keeps its
+    // unreachable cells; the last tile row's rows past W hold none either)
+    const bool own = own_lane<H, R, kSplit>(lane, wave, waves);
+    const int x0 = row0 + lane * R, left = (W + 7) / 8 * 8 - x0;
+    const TallPlanes<H, R> tiles{
+        reinterpret_cast<uint4*>(b.cost_tiles + agent_index * tiled_cells(W, H)) + x0 + 8, strip_cells(W) / 8u,
+        !own || left < 0 ? 0 : (left < R ? left : R)};
+    SearchPlanes<H, R, kFieldHigh> P;
+    uint32_t vis[N];
+    int overflow = 0;
+    P.tall = P.batches = 0;
+    if (ok) {
+        load_search_rows<H, R>(env_bits, W, x0, P.avail);
+        overflow = search_rows<H, R, kSplit, kFieldHigh, 0, true>(P, gx, gy, x0, lane, wave, waves, s, tiles);
+        // the reached cells (the goal's own is free): the free rows once more,
+        // which would otherwise be held through the search
+        load_search_rows<H, R>(env_bits, W, x0, vis);
+#pragma unroll
+        for (int i = 0; i < N; ++i) vis[i] &= ~P.avail[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            vis[i] = P.low[0][i] = P.low[1][i] = P.low[2][i] = 0;
+#pragma unroll
+            for (int p = 0; p < kFieldHigh; ++p) P.high[p][i] = 0;
+        }
+    }
+    uint32_t info = ok ? (uint32_t)(overflow < 0xFFFFFF ? overflow : 0xFFFFFF) << kInfoOverflowShift : kInfoBadGoal;
+    if ((uint32_t)spx < (uint32_t)W && (uint32_t)spy < (uint32_t)H) {
+        // cell 0: the agent's; 1..4: x - 1, x + 1, y - 1, y + 1; each as its
+        // reached bit and its level's bit 1 (0 off the map)
+        uint32_t cell[5];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) {
+            const int x = spx + (c == 2 ? 1 : 0) - (c == 1 ? 1 : 0), y = spy + (c == 4 ? 1 : 0) - (c == 3 ? 1 : 0);
+            const int at = x - row0, l = at / R;
+            uint32_t v = 0, p1 = 0;
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                if (at - l * R == i / HW && (y >> 5) == i % HW) {
+                    v = vis[i];
+                    p1 = P.low[0][i];
+                }
+            }
+            const bool here = at >= 0 && l < kWave && x < W && y >= 0 && y < H;
+            const int src = here ? l : 0;
+            v = (uint32_t)__builtin_amdgcn_readlane((int)v, src) >> (y & 31);
+            p1 = (uint32_t)__builtin_amdgcn_readlane((int)p1, src) >> (y & 31);
+            cell[c] = here ? (v & 1u) | (p1 & 1u) << 1 : 0u;
+            if (kSplit && here && own_lane<H, R, true>(l, wave, waves) && lane == 0) s.cell[c] = cell[c];
+        }
+        if (kSplit) {
+            // the owners' values (cells off the map have no owner)
+            lds_barrier();
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                const bool on = c == 0 || (c == 1 ? spx > 0 : (c == 2 ? spx + 1 < W : (c == 3 ? spy > 0 : spy + 1 < H)));
+                cell[c] = on ? (uint32_t)__builtin_amdgcn_readfirstlane((int)s.cell[c]) : 0u;
+            }
+        }
+        const uint32_t a01 = ((uint32_t)(spx + spy + gx + gy) ^ (cell[0] >> 1)) & 1u;
+#pragma unroll
+        for (int c = 1; c < 5; ++c) {
+            const uint32_t closer = (cell[0] & 1u) ? a01 ^ (cell[c] >> 1) : 1u;
+            info |= (cell[c] & closer & 1u) << (4 - c);
+        }
+    }
+    // marks, where every level is below 4,095: the closer reachable neighbours
+    // of every cell, bit-parallel (two reachable neighbours' levels differ by
+    // one), from the levels' two low bits
+    const bool marks = P.batches * 16 < (int)kMarkedMask;
+    if (marks) info |= kInfoMarked;
+    if (kSplit) meet_rows<H, R>(vis, P.low[0], lane, wave, waves, s);
+    // the tiles: 16 bits of every cell, every bit of an unreached cell set
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int r = i / HW, k = i % HW;
+        const uint32_t up = r > 0 ? vis[r > 0 ? i - HW : 0] : word_from_below(vis[(R - 1) * HW + k]);
+        const uint32_t up1 = r > 0 ? P.low[0][r > 0 ? i - HW : 0] : word_from_below(P.low[0][(R - 1) * HW + k]);
+        const uint32_t dn = r + 1 < R ? vis[r + 1 < R ? i + HW : 0] : word_from_above(vis[k]);
+        const uint32_t dn1 = r + 1 < R ? P.low[0][r + 1 < R ? i + HW : 0] : word_from_above(P.low[0][k]);
+        const uint32_t odd = ((x0 + r + gx + gy) & 1) ? 0x55555555u : 0xAAAAAAAAu;
+        const uint32_t par = vis[i] & odd, none = ~vis[i];
+        const uint32_t a01 = odd ^ P.low[0][i];
+        const int il = k > 0 ? i - 1 : 0, ir = k + 1 < HW ? i + 1 : 0;
+        const uint32_t lf = k > 0 ? __builtin_amdgcn_alignbit(vis[i], vis[il], 31) : vis[i] << 1;
+        const uint32_t lf1 = k > 0 ? __builtin_amdgcn_alignbit(P.low[0][i], P.low[0][il], 31) : P.low[0][i] << 1;
+        const uint32_t rt = k + 1 < HW ? __builtin_amdgcn_alignbit(vis[ir], vis[i], 1) : vis[i] >> 1;
+        const uint32_t rt1 = k + 1 < HW ? __builtin_amdgcn_alignbit(P.low[0][ir], P.low[0][i], 1) : P.low[0][i] >> 1;
+        // one word after the other: their loads and addresses side by side
+        // would take more registers than the search
+        asm volatile("" ::: "memory");
+        if (i / HW < tiles.valid) {
+            uint4* out = tiles.rows + (size_t)((i % HW) * 4 + 1) * tiles.strip_words + i / HW;
+            // level bits 4 and up: the register planes, then the tall ones
+            uint32_t t[12];
+#pragma unroll
+            for (int p = 0; p < 12; ++p) {
+                t[p] = 0;
+                if (p < kFieldHigh) t[p] = P.high[p < kFieldHigh ? p : 0][i];
+                else if (P.tall > p - kFieldHigh) t[p] = *tiles.word(p - kFieldHigh, i);
+            }
+            if (marks) {
+                t[8] = rt & (a01 ^ rt1);
+                t[9] = lf & (a01 ^ lf1);
+                t[10] = dn & (a01 ^ dn1);
+                t[11] = up & (a01 ^ up1);
+            }
+            asm volatile("" ::: "memory");  // read before their rows are written
+#pragma unroll 1
+            for (uint32_t q = 0; q < 4; ++q) {
+                const uint32_t unr = __builtin_amdgcn_perm(none, none, q * 0x01010101u);
+                const uint32_t l0 = gather_bytes(par, P.low[0][i], P.low[1][i], P.low[2][i], q) | unr;
+                const uint32_t l1 = gather_bytes(t[0], t[1], t[2], t[3], q) | unr;
+                const uint32_t h0 = gather_bytes(t[4], t[5], t[6], t[7], q) | unr;
+                const uint32_t h1 = gather_bytes(t[8], t[9], t[10], t[11], q) | unr;
+                const uint64_t lo = transpose8x8((uint64_t)l1 << 32 | l0);  // byte c: bits 0-7 of cell c
+                const uint64_t hi = transpose8x8((uint64_t)h1 << 32 | h0);  // byte c: bits 8-15
+                const uint32_t lo0 = (uint32_t)lo, lo1 = (uint32_t)(lo >> 32), hi0 = (uint32_t)hi, hi1 = (uint32_t)(hi >> 32);
+                out[q * tiles.strip_words] =
+                    make_uint4(__builtin_amdgcn_perm(hi0, lo0, 0x05010400u), __builtin_amdgcn_perm(hi0, lo0, 0x07030602u),
+                               __builtin_amdgcn_perm(hi1, lo1, 0x05010400u), __builtin_amdgcn_perm(hi1, lo1, 0x07030602u));
+            }
+        }
+    }
+    if (kSplit) lds_barrier();  // the exchange and s.cell are rewritten by the next refresh
     return info;
 }
 
 // ---------------------------------------------------------------------------
-// Pass 1a (maps of more than kMarkedCells cells): unpack + goal-cache refresh
-// + agent info, one lane per agent, no LDS.  An agent whose field is kept
-// gets its greedy mask from the tiled field; one whose reset flag is set is
-// marked for pass 1b.
+// Pass 1 on maps of more than kMarkedCells cells: unpack, goal-cache refresh,
+// agent info and the fields of changed goals, in one launch.  Workgroup g
+// unpacks agents [g * per_group, (g + 1) * per_group), one thread per agent
+// and pass; an agent whose field is kept gets its greedy mask from the tiled
+// field, one whose reset flag is set is listed in LDS.  Then the listed
+// fields are searched: by one wavefront each where a wavefront holds the
+// whole map (W <= 64 R), or (kSplit) by the whole workgroup one after the
+// other.  A build without a
+// changed goal is the unpack alone.
+//
+// The grid is the workgroups resident at once (field_waves_per_simd), or one
+// per wavefront's worth of agents, so that a batch of new fields covers the
+// chip: ranges rounded to whole passes of the workgroup's threads left 8,192
+// new fields to 64 (128 x 128) and 32 (256 x 256) workgroups.  Bound by VALU
+// issue when every field is new.  8,192 new fields of i.i.d. 128 x 128 maps
+// (14 k VALU wavefront instructions each, 0.18 ms of issue): 15.8 ms with a
+// workgroup of two wavefronts, a barrier and a 16-plane update per level ->
+// 0.25 ms; of 256 x 256 warehouses (109 k each, 1.5 ms of issue): 79.8 ->
+// 2.85 ms (3.26 with two workgroups per CU instead of three).  Without a
+// changed goal (131,072 agents, 256 x 256): 7.2 -> 6.8 us, 8.8 with the cross
+// of five cells read for every agent instead of its own cell's mark.
 // ---------------------------------------------------------------------------
-constexpr int kUnpackThreads = 256;
+constexpr int kFieldWaves = 4;  // wavefronts of a workgroup whose wavefronts search on their own
 
-template <int H, bool kRows>
-__global__ __launch_bounds__(kUnpackThreads) void unpack_kernel(
-    jl_mapfgpt_t b, const int16_t* __restrict__ raw_rows, const int16_t* __restrict__ cur_x,
-    const int16_t* __restrict__ cur_y, const int16_t* __restrict__ goal_x,
-    const int16_t* __restrict__ goal_y) {
-    const int N = b.n_envs * b.n_agents;
-    const int i = blockIdx.x * kUnpackThreads + threadIdx.x;
-    // the build's diagnostics start from zero; pass 2 and append_actions add
-    if (blockIdx.x == 0 && threadIdx.x < 4) b.diagnostics[threadIdx.x] = 0;
-    if (i >= N) return;
-    uint32_t info;
-    const uint4 st = unpack_agent<kRows>(b, i, raw_rows, cur_x, cur_y, goal_x, goal_y, info);
-    const uint32_t px = st.y & 0xFFFFu, py = st.y >> 16;
-    if ((st.w >> 16) != 0) {
-        info |= kInfoNeedsBfs;
-    } else if (px < (uint32_t)b.map_w && py < (uint32_t)H) {
-        info |= kept_greedy<H, false>(b, (size_t)i, (int)px, (int)py);
-    }
-    b.agent_info[i] = info;
+template <int H, int R, bool kSplit>
+constexpr int field_waves() {
+    return kSplit ? SearchShape<H, R>::kMaxWaves : kFieldWaves;
 }
 
-// ---------------------------------------------------------------------------
-// Pass 1b: BFS of the marked agents.  A fixed grid sized to the CUs the LDS
-// fields allow; wavefront g scans agents [g * per_wave, (g + 1) * per_wave)
-// for the mark, so a build without a changed goal costs one scan of
-// agent_info.  Each refresh completes the agent's info word.
-// ---------------------------------------------------------------------------
-template <int H, int R, int kWaves>
-__global__ __launch_bounds__(kWave* kWaves) void bfs_kernel(jl_mapfgpt_t b, int per_wave) {
-    extern __shared__ __align__(16) uint16_t s_dist_all[];
-    const int N = b.n_envs * b.n_agents;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    uint16_t* s_dist = s_dist_all + (size_t)wave * b.map_w * H;  // this wavefront's field
-    const int begin = (blockIdx.x * kWaves + wave) * per_wave;
-    const int end = (begin + per_wave) < N ? (begin + per_wave) : N;
-    for (int c0 = begin; c0 < end; c0 += kWave) {
-        const int i = c0 + lane;
-        const uint32_t mine = i < end ? b.agent_info[i] : 0u;
-        uint64_t todo = __ballot((mine & kInfoNeedsBfs) != 0);
-        while (todo) {
-            const int src = __ffsll((unsigned long long)todo) - 1;
-            todo &= todo - 1;
-            const size_t agent_index = (size_t)c0 + src;
-            // the agent's state row as pass 1a left it
-            const uint4 row = *reinterpret_cast<const uint4*>(b.state_packed + agent_index * 8);
-            const uint32_t bits = refresh_field<H, R, false>(
-                b, agent_index, row.x & 0xFFFFu, (int)(row.z & 0xFFFFu), (int)(row.z >> 16),
-                (int)(row.y & 0xFFFFu), (int)(row.y >> 16), s_dist);
-            if (lane == src) b.agent_info[agent_index] = (mine & ~(kInfoNeedsBfs | kInfoGreedy)) | bits;
-        }
-    }
-}
-
-// Pass 1 as one launch on maps of more than 64 rows (and more than
-// kMarkedCells cells): unpack_kernel's work and the BFS of the changed goals.
-// Workgroup g of R wavefronts unpacks agents [g * per_group, (g + 1) *
-// per_group), one thread per agent and pass, and lists those whose goal
-// changed (reset flag) in LDS; then the whole workgroup refreshes their
-// fields one after the other (refresh_field_group), and each agent's thread
-// completes its info word.  A build without a changed goal is the unpack
-// alone.  The grid is sized to the workgroups resident at once (the group
-// BFS's registers allow two per CU), so the unpack's round trips overlap.
-template <int H, int R, bool kRows>
-__global__ __launch_bounds__(kWave* R) void unpack_group_bfs_kernel(
+template <int H, int R, bool kSplit, bool kRows>
+__global__ __launch_bounds__((kWave * field_waves<H, R, kSplit>()))
+__attribute__((amdgpu_waves_per_eu(field_waves_per_simd<kSplit>()))) void unpack_fields_kernel(
     jl_mapfgpt_t b, const int16_t* __restrict__ raw_rows, const int16_t* __restrict__ cur_x,
     const int16_t* __restrict__ cur_y, const int16_t* __restrict__ goal_x,
-    const int16_t* __restrict__ goal_y, int per_group) {
-    constexpr int kThreads = kWave * R;
-    __shared__ uint64_t s_words[group_bfs_words<H, R>()];
-    __shared__ uint32_t s_gm[8];
+    const int16_t* __restrict__ goal_y, int per_group, int waves) {
+    __shared__ SearchLds<H, R, kSplit, true, field_waves<H, R, kSplit>()> s_search;
     __shared__ int s_n;
-    extern __shared__ __align__(16) uint4 s_list[];  // [per_group]: agent, state row words y, z
+    extern __shared__ __align__(16) uint4 s_list[];  // [per_group]: agent, info | env << 16, state row words y, z
     const int N = b.n_envs * b.n_agents;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int threads = waves * kWave;
     const int begin = blockIdx.x * per_group;
     const int end = (begin + per_group) < N ? (begin + per_group) : N;
     // the build's diagnostics start from zero; pass 2 and append_actions add
     if (blockIdx.x == 0 && tid < 4) b.diagnostics[tid] = 0;
     if (tid == 0) s_n = 0;
     __syncthreads();
-    for (int i = begin + tid; i < end; i += kThreads) {
+    for (int i = begin + tid; i < end; i += threads) {
         uint32_t info;
+        const uint32_t kept = b.agent_info[i] & kInfoMarked;
         const uint4 st = unpack_agent<kRows>(b, i, raw_rows, cur_x, cur_y, goal_x, goal_y, info);
         const uint32_t px = st.y & 0xFFFFu, py = st.y >> 16;
         if ((st.w >> 16) != 0) {
@@ -561,20 +602,22 @@ __global__ __launch_bounds__(kWave* R) void unpack_group_bfs_kernel(
             s_list[atomicAdd(&s_n, 1)] = make_uint4((uint32_t)i, info | (st.x << 16), st.y, st.z);
             continue;
         }
-        if (px < (uint32_t)b.map_w && py < (uint32_t)H) info |= kept_greedy<H, false>(b, (size_t)i, (int)px, (int)py);
+        info |= kept;
+        if (px < (uint32_t)b.map_w && py < (uint32_t)H) info |= kept_greedy<H>(b, (size_t)i, (int)px, (int)py, kept != 0);
         b.agent_info[i] = info;
     }
     __syncthreads();
     const int n = __builtin_amdgcn_readfirstlane(s_n);
-    for (int k = 0; k < n; ++k) {
+    for (int k = kSplit ? 0 : wave; k < n; k += kSplit ? 1 : kFieldWaves) {
         const uint4 it = s_list[k];
         const uint32_t agent = (uint32_t)__builtin_amdgcn_readfirstlane((int)it.x);
         const uint32_t head = (uint32_t)__builtin_amdgcn_readfirstlane((int)it.y);
         const uint32_t pos = (uint32_t)__builtin_amdgcn_readfirstlane((int)it.z);
         const uint32_t goal = (uint32_t)__builtin_amdgcn_readfirstlane((int)it.w);
-        const uint32_t bits = refresh_field_group<H, R>(b, agent, head >> 16, (int)(goal & 0xFFFFu), (int)(goal >> 16),
-                                                        (int)(pos & 0xFFFFu), (int)(pos >> 16), s_words, s_gm);
-        if (tid == 0) b.agent_info[agent] = (head & 0xFFFFu) | bits;
+        const uint32_t bits = refresh_field_rows<H, R, kSplit>(b, agent, head >> 16, (int)(goal & 0xFFFFu),
+                                                               (int)(goal >> 16), (int)(pos & 0xFFFFu),
+                                                               (int)(pos >> 16), wave, waves, s_search);
+        if (kSplit ? tid == 0 : lane == 0) b.agent_info[agent] = (head & 0xFFFFu) | bits;
     }
 }
 
@@ -588,8 +631,7 @@ __host__ __device__ inline size_t marked_wave_lds(int W, int H) {
 
 // ---------------------------------------------------------------------------
 // Pass 1 for maps of at most kMarkedCells cells (8 KB fields) when the
-// single-launch build does not apply: 1a and 1b in one launch, one lane per
-// agent and 4 wavefronts per workgroup, each wavefront refreshing the fields
+// single-launch build does not apply: one lane per agent and 4 wavefronts per workgroup, each wavefront refreshing the fields
 // of its own agents whose goal changed in its LDS field.  The tiled copies
 // it writes carry the greedy marks (jl_common.h, marked_fields).
 // ---------------------------------------------------------------------------
@@ -614,7 +656,7 @@ __global__ __launch_bounds__(kWave* kWaves) void unpack_bfs_kernel(
     const bool reset = i < N && (st.w >> 16) != 0;
     const uint32_t px = st.y & 0xFFFFu, py = st.y >> 16;
     if (i < N && !reset && px < (uint32_t)W && py < (uint32_t)H)
-        info |= kept_greedy<H, true>(b, (size_t)i, (int)px, (int)py);
+        info |= kept_greedy<H>(b, (size_t)i, (int)px, (int)py, true);
 
     uint64_t todo = __ballot(reset);
     while (todo) {
@@ -623,7 +665,7 @@ __global__ __launch_bounds__(kWave* kWaves) void unpack_bfs_kernel(
         const uint32_t sx = (uint32_t)__shfl((int)st.x, src, kWave);
         const uint32_t sy = (uint32_t)__shfl((int)st.y, src, kWave);
         const uint32_t sz = (uint32_t)__shfl((int)st.z, src, kWave);
-        const uint32_t bits = refresh_field<H, R, true>(
+        const uint32_t bits = refresh_field<H, R>(
             b, (size_t)(i - lane) + src, sx & 0xFFFFu, (int)(sz & 0xFFFFu), (int)(sz >> 16),
             (int)(sy & 0xFFFFu), (int)(sy >> 16), s_dist);
         if (lane == src) info |= bits;
@@ -862,9 +904,6 @@ __global__ __launch_bounds__(kTokThreads) void tokens_kernel(jl_mapfgpt_t b) {
     uint32_t* my_slots = reinterpret_cast<uint32_t*>(my_lds + kWinBytes + kRowBytes);
     constexpr int kTmplWords = kTmplBytes / 4;
     static_assert(kTmplBytes % 4 == 0, "template words");
-    // distance bits of a tiled field value: only maps of at most
-    // kMarkedCells cells, all of them dense here, carry greedy marks
-    const uint32_t fmask = kDense ? field_mask(W, H) : 0xFFFFu;
     // phase 1 at the highest priority; the ego loop lowers it as each
     // wavefront advances
     __builtin_amdgcn_s_setprio(3);
@@ -901,13 +940,15 @@ __global__ __launch_bounds__(kTokThreads) void tokens_kernel(jl_mapfgpt_t b) {
         const bool valid = px < (uint32_t)W && py < (uint32_t)H;
         // the byte offset of the first tile-row segment of the agent's
         // window from the env's first tiled field, bit 0 set when the window
-        // spans three column strips (an agent off the map: cell 0's window)
+        // spans three column strips (an agent off the map: cell 0's window),
+        // bit 1 when the field carries marks
         {
             const int ex = valid ? (int)px : 0, ey = valid ? (int)py : 0;
             const int tyl = ((ey - kRadius + 64) >> 3) - 8;  // floor((ey - 5) / 8)
             const bool third = (tyl + 2) * 8 <= ey + kRadius;
             s_seg[a] = (uint32_t)a * (uint32_t)tiled_cells(W, H) * 2u + (uint32_t)(tyl + 1) * strip_cells(W) * 2u +
-                       (uint32_t)(ex - kRadius + 8) * 16u + (third ? 1u : 0u);
+                       (uint32_t)(ex - kRadius + 8) * 16u + (third ? 1u : 0u) +
+                       (field_mask(W, H, info) == kMarkedMask ? 2u : 0u);
         }
         // the template: position (kNoAgent off the map: such an ego's row is
         // padding, and no window holds it), goal, history codes, greedy mask
@@ -1087,7 +1128,7 @@ __global__ __launch_bounds__(kTokThreads) void tokens_kernel(jl_mapfgpt_t b) {
     };
     // Cost token of a window value through the LDS table: index clamp(d - c +
     // 21, 0, 42) (42 below -20, 43 above +20) or 43 for an unreachable cell.
-    auto cost_token_lut = [&](uint32_t v, int c_minus_21) {
+    auto cost_token_lut = [&](uint32_t v, int c_minus_21, uint32_t fmask) {
         const int t = (int)(v & fmask) - c_minus_21;
         const int i = t < 0 ? 0 : (t > 2 * kCostLimit + 2 ? 2 * kCostLimit + 2 : t);
         return s_lut[v == kUnreachable ? kLutUnreachable : i];
@@ -1101,6 +1142,7 @@ __global__ __launch_bounds__(kTokThreads) void tokens_kernel(jl_mapfgpt_t b) {
             const int ex = (int)(pos & 0xFFFFu), ey = (int)(pos >> 16);
             // region row = dx + 5, column = dy + 5 + ((ey + 3) & 7) (see seg_load)
             const uint16_t* win = win_base + (rec.w >> 24);
+            const uint32_t fmask = (rec.z & 2u) ? kMarkedMask : 0xFFFFu;  // distance bits of the ego's field
             const uint32_t craw = win[kRadius * kRegionCols + kRadius];
             const uint32_t center = field_distance((uint32_t)__builtin_amdgcn_readfirstlane((int)craw), fmask);
             const uint32_t v0 = win[win0];  // raw tiled values: the table index strips the marks
@@ -1147,8 +1189,8 @@ __global__ __launch_bounds__(kTokThreads) void tokens_kernel(jl_mapfgpt_t b) {
             my_slots[0] = centre_id;
             // cost tokens
             const int c21 = (int)center - (kCostLimit + 1);
-            my_row[q0] = cost_token_lut(v0, c21);
-            my_row[q1] = cost_token_lut(v1, c21);
+            my_row[q0] = cost_token_lut(v0, c21, fmask);
+            my_row[q1] = cost_token_lut(v1, c21, fmask);
             wave_sync();
             // agent section: slots in use now or for the previous ego; a
             // slot at or past nsel is padding.  Up to six slots (tokens
@@ -1385,7 +1427,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(H <= 1
     const BuildLayout L = build_layout(A, W, H, kWaves);
     const size_t cells = (size_t)W * H;
     const size_t tcells = tiled_cells(W, H);
-    const uint32_t fmask = field_mask(W, H);
+    constexpr uint32_t fmask = kMarkedMask;
     uint16_t* s_map = reinterpret_cast<uint16_t*>(smem + L.map_off);
     int* s_tmpl = reinterpret_cast<int*>(smem + L.tmpl_off);
     int* s_lut = reinterpret_cast<int*>(smem + L.lut_off);
@@ -1486,7 +1528,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(H <= 1
             const uint32_t sx = (uint32_t)__builtin_amdgcn_readfirstlane((int)it.y);
             const uint32_t pos = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_rec[a * kBuildRecWords]);
             const uint32_t goal = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_rec[a * kBuildRecWords + 1]);
-            const uint32_t bits = refresh_field<H, R, true, false>(
+            const uint32_t bits = refresh_field<H, R, false>(
                 b, (size_t)env * A + a, sx & 0xFFFFu, (int)(goal & 0xFFFFu), (int)(goal >> 16),
                 (int)(pos & 0xFFFFu), (int)(pos >> 16), s_dist);
             if (lane == 0) s_info[a] |= bits;
@@ -1495,7 +1537,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(H <= 1
         const int nround = (nlist - r0) < L.bfs_waves ? (nlist - r0) : L.bfs_waves;
         for (int f = 0; f < nround; ++f) {
             const uint32_t a = s_list[r0 + f].x;
-            store_field_tiles<H, true>(b, (size_t)env * A + a, reinterpret_cast<uint16_t*>(smem) + (size_t)f * cells,
+            store_field_tiles<H>(b, (size_t)env * A + a, reinterpret_cast<uint16_t*>(smem) + (size_t)f * cells,
                                        tid, kThreads);
         }
         // the refreshed fields are stored before any window load of this
@@ -1583,7 +1625,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(H <= 1
         // unreachable)
         uint32_t greedy = inf & kInfoGreedy;
         if (!reset && valid)
-            greedy = f_center != kUnreachable ? f_center >> 12 : kept_greedy<H, false>(b, g, (int)px, (int)py);
+            greedy = f_center != kUnreachable ? f_center >> 12 : kept_greedy<H>(b, g, (int)px, (int)py, true);
         tp[9] = copy_token(greedy, 5);
     }
     // wavefront sums, then one LDS add per wavefront and counter
@@ -1860,7 +1902,6 @@ __global__ __launch_bounds__(256) void agent_at_cell_kernel(jl_mapfgpt_t b) {
 template <int H>
 __global__ __launch_bounds__(256) void cost_to_go_kernel(jl_mapfgpt_t b) {
     const int W = b.map_w;
-    const uint32_t fmask = field_mask(W, H);
     const size_t fields = (size_t)b.n_envs * b.n_agents;
     const size_t per_field = (size_t)W * (H / 8);  // 16-byte words of a row-major field
     const size_t total = fields * per_field;
@@ -1872,6 +1913,7 @@ __global__ __launch_bounds__(256) void cost_to_go_kernel(jl_mapfgpt_t b) {
         const size_t f = i / per_field;
         const uint32_t w = (uint32_t)(i - f * per_field);
         const uint32_t x = w / (H / 8), y8 = w - x * (H / 8);  // row, 8-cell group
+        const uint32_t fmask = field_mask(W, H, marked_fields(W, H) ? 0u : b.agent_info[f]);
         v4i v = tiles[f * (tcells / 8) + (y8 + 1) * strip_words + x + 8];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -1924,11 +1966,26 @@ int check_builder(const jl_mapfgpt_t* b) {
 }
 
 
-// Pass 1b wavefronts per workgroup: each owns a W*H uint16 LDS field; up to
-// 64 KB of them per workgroup, at most 4.
-inline int pass1_waves(int W, int H) {
-    const size_t field = (size_t)W * H * 2;
-    return field <= 16384 ? 4 : (field <= 32768 ? 2 : 1);
+// Pass 1 of unmarked maps: R rows per lane, the wavefronts on their own or
+// (kSplit) one field per workgroup.
+template <int H, int R, bool kSplit, bool kRows>
+int launch_fields(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx, const int16_t* cy,
+                  const int16_t* gx, const int16_t* gy, hipStream_t stream) {
+    const int N = b->n_envs * b->n_agents;
+    const int waves = kSplit ? split_waves<H, R>(b->map_w) : kFieldWaves;
+    // every workgroup that is resident at once, each with a field per
+    // searching wavefront (or workgroup) at least
+    const int resident = device_cus() * (4 * field_waves_per_simd<kSplit>() / waves);
+    const int per = kSplit ? 1 : kFieldWaves;
+    int groups = (N + per - 1) / per;
+    if (groups > resident) groups = resident;
+    constexpr int kMaxList = 1024;  // 16 KB of LDS list per workgroup
+    if ((N + groups - 1) / groups > kMaxList) groups = (N + kMaxList - 1) / kMaxList;
+    const int per_group = ((N + groups - 1) / groups + per - 1) / per * per;
+    hipLaunchKernelGGL((unpack_fields_kernel<H, R, kSplit, kRows>), dim3((N + per_group - 1) / per_group),
+                       dim3(kWave * waves), (size_t)per_group * sizeof(uint4), stream, *b, rows, cx, cy, gx, gy,
+                       per_group, waves);
+    return launch_status();
 }
 
 template <int H, int R, bool kRows>
@@ -1944,45 +2001,12 @@ int launch_pass1(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx, 
                            *b, rows, cx, cy, gx, gy);
         return launch_status();
     }
-    if constexpr (R > 1) {
-        // unpack and the changed goals' fields in one launch: two workgroups
-        // of R wavefronts per CU (the group BFS's registers), each over a
-        // whole number of passes of its threads
-        const int max_groups = (N + kWave * R - 1) / (kWave * R);
-        int groups = device_cus() * 2;
-        if (groups > max_groups) groups = max_groups;
-        constexpr int kMaxList = 3072;  // 48 KB of LDS list per workgroup
-        if ((N + groups - 1) / groups > kMaxList) groups = (N + kMaxList - 1) / kMaxList;
-        const int per_group = ((N + groups - 1) / groups + kWave * R - 1) / (kWave * R) * (kWave * R);
-        hipLaunchKernelGGL((unpack_group_bfs_kernel<H, R, kRows>), dim3((N + per_group - 1) / per_group),
-                           dim3(kWave * R), (size_t)per_group * sizeof(uint4), stream, *b, rows, cx, cy, gx, gy,
-                           per_group);
-        return launch_status();
-    }
-    hipLaunchKernelGGL((unpack_kernel<H, kRows>), dim3((N + kUnpackThreads - 1) / kUnpackThreads),
-                       dim3(kUnpackThreads), 0, stream, *b, rows, cx, cy, gx, gy);
-    int rc = launch_status();
-    if (rc) return rc;
-    const int waves = pass1_waves(b->map_w, H);
-    const size_t lds = (size_t)waves * b->map_w * H * sizeof(uint16_t);
-    const int per_cu = (int)(160 * 1024 / lds) < 8 ? (int)(160 * 1024 / lds) : 8;
-    // whole-wavefront ranges of at least one wavefront of agents
-    const int max_waves = (N + kWave - 1) / kWave;
-    int total_waves = device_cus() * (per_cu > 0 ? per_cu : 1) * waves;
-    if (total_waves > max_waves) total_waves = max_waves;
-    const int per_wave = ((N + total_waves - 1) / total_waves + kWave - 1) / kWave * kWave;
-    const int blocks = ((N + per_wave - 1) / per_wave + waves - 1) / waves;
-    if (waves == 4) {
-        hipLaunchKernelGGL((bfs_kernel<H, R, 4>), dim3(blocks), dim3(kWave * 4), lds, stream, *b,
-                           per_wave);
-    } else if (waves == 2) {
-        hipLaunchKernelGGL((bfs_kernel<H, R, 2>), dim3(blocks), dim3(kWave * 2), lds, stream, *b,
-                           per_wave);
-    } else {
-        hipLaunchKernelGGL((bfs_kernel<H, R, 1>), dim3(blocks), dim3(kWave), lds, stream, *b,
-                           per_wave);
-    }
-    return launch_status();
+    // a wavefront searches alone where a map's rows fit its lanes' registers
+    // (at most 8 words per lane), else the map's rows are split
+    constexpr int kAlone = SearchShape<H, 4>::N <= 8 ? 4 : (SearchShape<H, 2>::N <= 8 ? 2 : 1);
+    if constexpr (kWave * R * H <= kMarkedCells) return JL_ERR_PROFILE;  // always marked
+    else if constexpr (R <= kAlone) return launch_fields<H, R, false, kRows>(b, rows, cx, cy, gx, gy, stream);
+    else return launch_fields<H, kAlone, true, kRows>(b, rows, cx, cy, gx, gy, stream);
 }
 
 // The whole build runs as one launch (build_kernel) on maps of at most
