@@ -1,138 +1,169 @@
 // jl_energy.hip - uint8 "energy" BFS fields for the MAGAT builder on gfx950.
 //
-// One wavefront serves 64 consecutive jobs: it ballots the jobs that need a
-// field and runs the bit-parallel BFS (jl_bfs.h) for each, capped at 254
-// levels like generate_energy_map_kernel (energy_map.cu:174), staging the
-// distances in LDS and storing 255-d with 16-byte coalesced writes.  The
-// reference launches one 128-thread block per row whether or not its row
-// needs a refresh (energy_map.cu:262-271) and finds the changed rows with a
-// host-synchronised cumsum (grid_world_simulator.cpp:707-753); here the
-// incremental derived state is one launch on small maps (the scan, the
-// packed rows and the fields of changed goals: goal_changed_refresh_kernel).
+// A field is one row search (jl_bfs.h) capped at 255 levels, as
+// generate_energy_map_kernel's is (energy_map.cu:174), by one wavefront where
+// the map fits one, else by a workgroup; 255 - d leaves as 16-byte row
+// segments, its eight bits from the search's level planes by one 8x8 bit
+// transpose per 8 cells.  Jobs are dealt out in short runs to wavefronts (or
+// workgroups) all over the chip, and a run's jobs that need a field are
+// balloted.  The reference launches one 128-thread block per
+// row whether or not its row needs a refresh (energy_map.cu:262-271) and
+// finds the changed rows with a host-synchronised cumsum
+// (grid_world_simulator.cpp:707-753); here the incremental derived state is
+// one launch on small maps (the scan, the packed rows and the fields of
+// changed goals: goal_changed_refresh_kernel).
+//
+// Bound by VALU issue when every field is new.  16,000 fields of i.i.d.
+// 128 x 128 maps: 6.46 -> 0.34 ms (before: one wavefront per 64 jobs, one
+// after the other, with an LDS write per cell and level); 131,072 of 64 x 64:
+// 2.00 -> 0.40 ms.
 #include "jl_bfs.h"
 #include "jl_common.h"
 
 namespace jl {
 namespace {
 
-constexpr int kEnergyCap = 254;
+constexpr int kEnergyHigh = 4;     // register planes of level bits 4..7: all of a level below 256
+constexpr int kEnergyBatches = 16;  // 16 levels each
+constexpr int kEnergyWaves = 4;    // wavefronts of a workgroup whose wavefronts search on their own
 
-// One field by one wavefront (its LDS orderings are the wavefront's own, so
-// several wavefronts of a workgroup may run fields side by side).
-template <int H, int R>
-__device__ void energy_field(const uint32_t* __restrict__ env_bits, int W, int gx, int gy,
-                             uint8_t* s_dist, uint8_t* __restrict__ out) {
-    constexpr int HW = RowWords<H>::HW;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int cells = W * H;
-    for (int c = lane; c < cells; c += kWave) s_dist[c] = 255;
-    wave_sync();
-    uint64_t fr[R][HW];
-    load_free_rows<H, R>(env_bits, W, fr);
-    if (lane == 0) s_dist[gx * H + gy] = 0;
-    wave_sync();
-    wave_bfs<H, R, uint8_t>(fr, gx, gy, kEnergyCap, s_dist);
-    wave_sync();
-    const uint4* src = reinterpret_cast<const uint4*>(s_dist);
-    uint4* dst = reinterpret_cast<uint4*>(out);
-    for (int c = lane; c < cells / 16; c += kWave) {
-        uint4 v = src[c];
-        uint32_t* w = reinterpret_cast<uint32_t*>(&v);
+template <int H, int R, bool kSplit>
+constexpr int energy_waves() {
+    return kSplit ? SearchShape<H, R>::kMaxWaves : kEnergyWaves;
+}
+
+template <int H, int R, bool kSplit, int kWaves = energy_waves<H, R, kSplit>()>
+using EnergyLds = SearchLds<H, R, kSplit, false, kWaves>;
+
+// One field by the calling wavefront (kSplit: the workgroup, each wavefront on
+// its rows); every lane calls it with uniform arguments, the goal on the map.
+template <int H, int R, bool kSplit, typename Lds>
+__device__ __forceinline__ void energy_field(const uint32_t* __restrict__ env_bits, int W, int gx, int gy,
+                                             uint8_t* __restrict__ out, int wave, int waves, Lds& s) {
+    using S = SearchShape<H, R>;
+    constexpr int HW = S::HW, N = S::N;
+    // (taken afresh for every field: the addresses that follow from it would
+    // otherwise be held across the search)
+    int lane = threadIdx.x & (kWave - 1);
+    asm volatile("" : "+v"(lane));
+    const int x0 = (kSplit ? wave * S::kStep : 0) + lane * R;
+    SearchPlanes<H, R, kEnergyHigh> P;
+    load_search_rows<H, R>(env_bits, W, x0, P.avail);
+    search_rows<H, R, kSplit, kEnergyHigh, kEnergyBatches, false>(P, gx, gy, x0, lane, wave, waves, s, NoTallPlanes{});
+    uint32_t vis[N];
+    load_search_rows<H, R>(env_bits, W, x0, vis);
+    const bool own = own_lane<H, R, kSplit>(lane, wave, waves);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            uint32_t o = 0;
+    for (int i = 0; i < N; ++i) {
+        const int x = x0 + i / HW, k = i % HW;
+        // reached cells, the goal's own included where it is an obstacle
+        const uint32_t v = (vis[i] & ~P.avail[i]) | (x == gx && k == (gy >> 5) ? 1u << (gy & 31) : 0u);
+        // bits of 255 - d: each level bit inverted, none of an unreached cell
+        const uint32_t e0 = v & (((x + gx + gy) & 1) ? 0xAAAAAAAAu : 0x55555555u);
+        asm volatile("" ::: "memory");  // one word after the other (registers)
+        if (own && x < W) {
+            uint4* row = reinterpret_cast<uint4*>(out + (size_t)x * H + k * 32);
+#pragma unroll 1
+            for (uint32_t h = 0; h < 2; ++h) {
+                uint64_t b[2];
 #pragma unroll
-            for (int byte = 0; byte < 4; ++byte) {
-                const uint32_t d = (w[k] >> (8 * byte)) & 0xFFu;
-                o |= (d == 255u ? 0u : 255u - d) << (8 * byte);
+                for (uint32_t q = 0; q < 2; ++q) {
+                    const uint32_t lo = gather_bytes(e0, v & ~P.low[0][i], v & ~P.low[1][i], v & ~P.low[2][i], 2 * h + q);
+                    const uint32_t hi = gather_bytes(v & ~P.high[0][i], v & ~P.high[1][i], v & ~P.high[2][i],
+                                                     v & ~P.high[3][i], 2 * h + q);
+                    b[q] = transpose8x8((uint64_t)hi << 32 | lo);
+                }
+                row[h] = make_uint4((uint32_t)b[0], (uint32_t)(b[0] >> 32), (uint32_t)b[1], (uint32_t)(b[1] >> 32));
             }
-            w[k] = o;
         }
-        dst[c] = v;
     }
-    wave_sync();
+    if (kSplit) lds_barrier();  // the exchange is rewritten by the next field
+}
+
+// This wavefront's (kSplit: this workgroup's) run of `per` jobs of `count`.
+template <bool kSplit>
+__device__ __forceinline__ int run_begin(int per, int wave) {
+    return (kSplit ? (int)blockIdx.x : (int)blockIdx.x * kEnergyWaves + wave) * per;
 }
 
 // Jobs are state rows (launch_energy_map_kernel semantics).
-template <int H, int R>
-__global__ __launch_bounds__(kWave) void energy_rows_kernel(const uint32_t* __restrict__ grid_bits,
-                                                             uint8_t* __restrict__ energy,
-                                                             const uint16_t* __restrict__ states,
-                                                             int length, int E, int A, int W,
-                                                             int incremental_only) {
-    extern __shared__ uint8_t s_dist[];
+template <int H, int R, bool kSplit>
+__global__ __launch_bounds__((kWave * energy_waves<H, R, kSplit>())) void energy_rows_kernel(
+    const uint32_t* __restrict__ grid_bits, uint8_t* __restrict__ energy, const uint16_t* __restrict__ states,
+    int length, int E, int A, int W, int incremental_only, int per, int waves) {
+    __shared__ EnergyLds<H, R, kSplit> s_search;
     const int lane = threadIdx.x & (kWave - 1);
-    const int b = blockIdx.x * kWave + lane;
-    bool run = false;
-    uint32_t env = 0, agent = 0, gx = 0, gy = 0;
-    if (b < length) {
-        const uint4 r = *reinterpret_cast<const uint4*>(states + (size_t)b * 8);
-        env = r.x & 0xFFFFu;
-        agent = r.x >> 16;
-        gx = r.z & 0xFFFFu;
-        gy = r.z >> 16;
-        const uint32_t reset = r.w >> 16;
-        run = !(incremental_only && reset == 0) && env < (uint32_t)E && agent < (uint32_t)A &&
-              gx < (uint32_t)W && gy < (uint32_t)H;
-    }
-    uint64_t todo = __ballot(run);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const size_t cells = (size_t)W * H;
-    const int words = W * H / 32;
-    while (todo) {
-        const int src = __ffsll((unsigned long long)todo) - 1;
-        todo &= todo - 1;
-        const int e = __shfl((int)env, src, kWave);
-        const int a = __shfl((int)agent, src, kWave);
-        const int x = __shfl((int)gx, src, kWave);
-        const int y = __shfl((int)gy, src, kWave);
-        energy_field<H, R>(grid_bits + (size_t)e * words, W, x, y, s_dist,
-                           energy + ((size_t)e * A + a) * cells);
+    const int begin = run_begin<kSplit>(per, wave);
+    const int end = begin + per < length ? begin + per : length;
+    for (int c0 = begin; c0 < end; c0 += kWave) {
+        const int b = c0 + lane;
+        bool run = false;
+        uint32_t env = 0, agent = 0, gx = 0, gy = 0;
+        if (b < end) {
+            const uint4 r = *reinterpret_cast<const uint4*>(states + (size_t)b * 8);
+            env = r.x & 0xFFFFu;
+            agent = r.x >> 16;
+            gx = r.z & 0xFFFFu;
+            gy = r.z >> 16;
+            const uint32_t reset = r.w >> 16;
+            run = !(incremental_only && reset == 0) && env < (uint32_t)E && agent < (uint32_t)A &&
+                  gx < (uint32_t)W && gy < (uint32_t)H;
+        }
+        for (uint64_t todo = __ballot(run); todo; todo &= todo - 1) {
+            const int src = __builtin_ctzll(todo);
+            const int e = __builtin_amdgcn_readlane((int)env, src), a = __builtin_amdgcn_readlane((int)agent, src);
+            const int x = __builtin_amdgcn_readlane((int)gx, src), y = __builtin_amdgcn_readlane((int)gy, src);
+            energy_field<H, R, kSplit>(grid_bits + (size_t)e * (cells / 32), W, x, y,
+                                       energy + ((size_t)e * A + a) * cells, wave, waves, s_search);
+        }
     }
 }
 
 // Jobs are simulator agents whose goal_changed flag is set (or all).
-template <int H, int R>
-__global__ __launch_bounds__(kWave) void energy_flagged_kernel(jl_sim_t s, uint8_t* __restrict__ energy,
-                                                                int all_agents,
-                                                                const int64_t* __restrict__ prefix,
-                                                                uint16_t* __restrict__ changed) {
-    extern __shared__ uint8_t s_dist[];
+template <int H, int R, bool kSplit>
+__global__ __launch_bounds__((kWave * energy_waves<H, R, kSplit>())) void energy_flagged_kernel(
+    jl_sim_t s, uint8_t* __restrict__ energy, int all_agents, const int64_t* __restrict__ prefix,
+    uint16_t* __restrict__ changed, int per, int waves) {
+    __shared__ EnergyLds<H, R, kSplit> s_search;
     const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int A = s.n_agents, W = s.map_w;
     const int N = s.n_envs * A;
     // the scan's total: no goal changed, no field and no row to write
     if (!all_agents && prefix && prefix[N - 1] == 0) return;
-    const int g = blockIdx.x * kWave + lane;
-    bool run = false;
-    uint32_t gx = 0, gy = 0;
-    if (g < N) {
-        gx = s.goal_x[g];
-        gy = s.goal_y[g];
-        const bool flagged = s.goal_changed[g] != 0;
-        run = (all_agents || flagged) && gx < (uint32_t)W && gy < (uint32_t)H;
-        if (!all_agents && flagged && prefix && changed) {
-            const int64_t slot = prefix[g] - 1;
-            const uint32_t e = (uint32_t)(g / A), a = (uint32_t)(g - (int)e * A);
-            uint4 v;
-            v.x = (e & 0xFFFFu) | (a << 16);
-            v.y = (uint32_t)s.cur_x[g] | ((uint32_t)s.cur_y[g] << 16);
-            v.z = gx | (gy << 16);
-            v.w = (uint32_t)s.actions[g] | (1u << 16);
-            *reinterpret_cast<uint4*>(changed + slot * 8) = v;
-        }
-    }
-    uint64_t todo = __ballot(run);
     const size_t cells = (size_t)W * H;
-    const int words = W * H / 32;
-    while (todo) {
-        const int src = __ffsll((unsigned long long)todo) - 1;
-        todo &= todo - 1;
-        const int x = __shfl((int)gx, src, kWave);
-        const int y = __shfl((int)gy, src, kWave);
-        const int gi = blockIdx.x * kWave + src;
-        const int e = gi / A;
-        energy_field<H, R>(s.grid_bits + (size_t)e * words, W, x, y, s_dist,
-                           energy + (size_t)gi * cells);
+    const int begin = run_begin<kSplit>(per, wave);
+    const int end = begin + per < N ? begin + per : N;
+    for (int c0 = begin; c0 < end; c0 += kWave) {
+        const int g = c0 + lane;
+        bool run = false;
+        uint32_t gx = 0, gy = 0;
+        if (g < end) {
+            gx = s.goal_x[g];
+            gy = s.goal_y[g];
+            const bool flagged = s.goal_changed[g] != 0;
+            run = (all_agents || flagged) && gx < (uint32_t)W && gy < (uint32_t)H;
+            if (!all_agents && flagged && prefix && changed && (!kSplit || wave == 0)) {
+                const int64_t slot = prefix[g] - 1;
+                const uint32_t e = (uint32_t)(g / A), a = (uint32_t)(g - (int)e * A);
+                uint4 v;
+                v.x = (e & 0xFFFFu) | (a << 16);
+                v.y = (uint32_t)s.cur_x[g] | ((uint32_t)s.cur_y[g] << 16);
+                v.z = gx | (gy << 16);
+                v.w = (uint32_t)s.actions[g] | (1u << 16);
+                *reinterpret_cast<uint4*>(changed + slot * 8) = v;
+            }
+        }
+        for (uint64_t todo = __ballot(run); todo; todo &= todo - 1) {
+            const int src = __builtin_ctzll(todo);
+            const int x = __builtin_amdgcn_readlane((int)gx, src), y = __builtin_amdgcn_readlane((int)gy, src);
+            const int gi = c0 + src;
+            const int e = gi / A;
+            energy_field<H, R, kSplit>(s.grid_bits + (size_t)e * (cells / 32), W, x, y, energy + (size_t)gi * cells,
+                                       wave, waves, s_search);
+        }
     }
 }
 
@@ -146,8 +177,8 @@ __global__ __launch_bounds__(kWave) void energy_flagged_kernel(jl_sim_t s, uint8
 // at or past the total are cleared, so every row is written once without
 // ordering between workgroups (grid_world_simulator.cpp:709-733,
 // pack_changed_agent_state_kernel, 128_agents_map_step.cu:469-511).  Then
-// each wavefront runs the energy BFS of its changed agents in its own LDS
-// field (energy_map.cu:80-272).
+// each wavefront runs the energy BFS of its changed agents
+// (energy_map.cu:80-272).
 constexpr int kRefreshThreads = 1024;
 constexpr int kRefreshWaves = kRefreshThreads / kWave;
 constexpr int kRefreshGroups = 128;
@@ -157,10 +188,11 @@ __global__ __launch_bounds__(kRefreshThreads) void goal_changed_refresh_kernel(j
                                                                             int64_t* __restrict__ prefix,
                                                                             int64_t* __restrict__ count,
                                                                             uint16_t* __restrict__ changed) {
-    extern __shared__ uint8_t s_fields[];  // one W*H field per wavefront
+    __shared__ EnergyLds<H, 1, false, kRefreshWaves> s_search;
     __shared__ int64_t s_before[kRefreshWaves];
     __shared__ int64_t s_all[kRefreshWaves];
     __shared__ uint32_t s_scan[kRefreshWaves];
+    __shared__ uint32_t s_goal[kRefreshThreads];  // (held in LDS: the search leaves no registers for it)
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // uniform per wavefront
     const int A = s.n_agents, W = s.map_w;
@@ -200,6 +232,7 @@ __global__ __launch_bounds__(kRefreshThreads) void goal_changed_refresh_kernel(j
         const uint32_t t = __shfl_up(incl, off, kWave);
         if (lane >= off) incl += t;
     }
+    s_goal[tid] = gx | (gy << 16);
     if (lane == 0) {
         s_before[wave] = (int64_t)before;
         s_all[wave] = (int64_t)all;
@@ -233,19 +266,86 @@ __global__ __launch_bounds__(kRefreshThreads) void goal_changed_refresh_kernel(j
     }
     // the energy fields of this wavefront's changed agents
     const int cells = W * H;
-    uint64_t todo = __ballot(v != 0 && gx < (uint32_t)W && gy < (uint32_t)H);
-    uint8_t* s_dist = s_fields + (size_t)wave * cells;
-    while (todo) {
-        const int src = __ffsll((unsigned long long)todo) - 1;
-        todo &= todo - 1;
-        const int x = __shfl((int)gx, src, kWave);
-        const int y = __shfl((int)gy, src, kWave);
+    for (uint64_t todo = __ballot(v != 0 && gx < (uint32_t)W && gy < (uint32_t)H); todo; todo &= todo - 1) {
+        const int src = __builtin_ctzll(todo);
+        const uint32_t goal = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_goal[wave * kWave + src]);
+        const int x = (int)(goal & 0xFFFFu), y = (int)(goal >> 16);
         const int gi = c0 + wave * kWave + src;
         const int e = gi / A;
-        energy_field<H, 1>(s.grid_bits + (size_t)e * (cells / 32), W, x, y, s_dist,
-                           energy + (size_t)gi * cells);
+        energy_field<H, 1, false>(s.grid_bits + (size_t)e * (cells / 32), W, x, y, energy + (size_t)gi * cells, wave,
+                                  kRefreshWaves, s_search);
     }
 }
+
+// Workgroups and jobs per run.  A launch that makes every job's field is dealt
+// out in runs of about a quarter of what a resident wavefront (kSplit:
+// workgroup) does in all, so that the hardware evens out their lengths; one
+// that looks for the few changed goals, in one run per resident wavefront.
+struct EnergyGrid {
+    int groups, per, waves;
+};
+template <int H, int R, bool kSplit>
+EnergyGrid energy_grid(int jobs, int W, bool every) {
+    EnergyGrid g;
+    g.waves = kSplit ? split_waves<H, R>(W) : kEnergyWaves;
+    const int runs_per_group = kSplit ? 1 : kEnergyWaves;
+    constexpr int kPerCu = SearchShape<H, R>::N < 8 ? 16 : 12;  // resident wavefronts
+    int runs = device_cus() * (kPerCu / g.waves) * runs_per_group * (every ? 4 : 1);
+    if (runs > jobs) runs = jobs;
+    g.per = (jobs + runs - 1) / runs;
+    runs = (jobs + g.per - 1) / g.per;
+    g.groups = (runs + runs_per_group - 1) / runs_per_group;
+    return g;
+}
+
+// f.template operator()<R, kSplit>() with the lane layout of a W x H map: a
+// wavefront on its own where its lanes' registers hold the rows (at most 8
+// words each), else the map split over a workgroup.
+template <int H, typename F>
+int with_energy_layout(int W, F f) {
+    constexpr int kAlone = SearchShape<H, 4>::N <= 8 ? 4 : (SearchShape<H, 2>::N <= 8 ? 2 : 1);
+    if (W <= kWave) return f.template operator()<1, false>();
+    if constexpr (kAlone >= 2) {
+        if (W <= 2 * kWave) return f.template operator()<2, false>();
+        if constexpr (kAlone == 4) return f.template operator()<4, false>();
+        else return f.template operator()<2, true>();
+    } else {
+        return f.template operator()<1, true>();
+    }
+}
+
+template <int H>
+struct LaunchRows {
+    const uint32_t* grid_bits;
+    uint8_t* energy;
+    const uint16_t* states;
+    int length, n_envs, n_agents, map_w, incremental_only;
+    hipStream_t stream;
+    template <int R, bool kSplit>
+    int operator()() const {
+        const EnergyGrid g = energy_grid<H, R, kSplit>(length, map_w, !incremental_only);
+        hipLaunchKernelGGL((energy_rows_kernel<H, R, kSplit>), dim3(g.groups), dim3(kWave * g.waves), 0, stream,
+                           grid_bits, energy, states, length, n_envs, n_agents, map_w, incremental_only, g.per, g.waves);
+        return launch_status();
+    }
+};
+
+template <int H>
+struct LaunchFlagged {
+    const jl_sim_t* s;
+    uint8_t* energy;
+    int all_agents;
+    const int64_t* prefix;
+    uint16_t* changed;
+    hipStream_t stream;
+    template <int R, bool kSplit>
+    int operator()() const {
+        const EnergyGrid g = energy_grid<H, R, kSplit>(s->n_envs * s->n_agents, s->map_w, all_agents != 0);
+        hipLaunchKernelGGL((energy_flagged_kernel<H, R, kSplit>), dim3(g.groups), dim3(kWave * g.waves), 0, stream, *s,
+                           energy, all_agents, prefix, changed, g.per, g.waves);
+        return launch_status();
+    }
+};
 
 }  // namespace
 }  // namespace jl
@@ -259,24 +359,11 @@ extern "C" int jl_energy_maps(const uint32_t* grid_bits, uint8_t* energy, const 
     if (length == 0) return JL_OK;
     if (!states) return JL_ERR_ARG;
     if (!profile_ok(map_w, map_h)) return JL_ERR_PROFILE;
-    const int grid = (length + kWave - 1) / kWave;
-    const size_t lds = (size_t)map_w * map_h;
     JL_DISPATCH_H(map_h, {
-        if (map_w <= 64) {
-            hipLaunchKernelGGL((energy_rows_kernel<H, 1>), dim3(grid), dim3(kWave), lds,
-                               (hipStream_t)stream, grid_bits, energy, states, length, n_envs,
-                               n_agents, map_w, incremental_only);
-        } else if (map_w <= 128) {
-            hipLaunchKernelGGL((energy_rows_kernel<H, 2>), dim3(grid), dim3(kWave), lds,
-                               (hipStream_t)stream, grid_bits, energy, states, length, n_envs,
-                               n_agents, map_w, incremental_only);
-        } else {
-            hipLaunchKernelGGL((energy_rows_kernel<H, 4>), dim3(grid), dim3(kWave), lds,
-                               (hipStream_t)stream, grid_bits, energy, states, length, n_envs,
-                               n_agents, map_w, incremental_only);
-        }
+        return with_energy_layout<H>(map_w, LaunchRows<H>{grid_bits, energy, states, length, n_envs, n_agents, map_w,
+                                                          incremental_only, (hipStream_t)stream});
     });
-    return launch_status();
+    return JL_ERR_PROFILE;
 }
 
 extern "C" int jl_energy_maps_flagged(const jl_sim_t* s, uint8_t* energy, int32_t all_agents,
@@ -286,25 +373,11 @@ extern "C" int jl_energy_maps_flagged(const jl_sim_t* s, uint8_t* energy, int32_
         return JL_ERR_ARG;
     if (s->n_envs <= 0 || s->n_agents <= 0) return JL_ERR_ARG;
     if (!profile_ok(s->map_w, s->map_h)) return JL_ERR_PROFILE;
-    const int N = s->n_envs * s->n_agents;
-    const int grid = (N + kWave - 1) / kWave;
-    const size_t lds = (size_t)s->map_w * s->map_h;
     JL_DISPATCH_H(s->map_h, {
-        if (s->map_w <= 64) {
-            hipLaunchKernelGGL((energy_flagged_kernel<H, 1>), dim3(grid), dim3(kWave), lds,
-                               (hipStream_t)stream, *s, energy, all_agents, changed_prefix,
-                               changed_states);
-        } else if (s->map_w <= 128) {
-            hipLaunchKernelGGL((energy_flagged_kernel<H, 2>), dim3(grid), dim3(kWave), lds,
-                               (hipStream_t)stream, *s, energy, all_agents, changed_prefix,
-                               changed_states);
-        } else {
-            hipLaunchKernelGGL((energy_flagged_kernel<H, 4>), dim3(grid), dim3(kWave), lds,
-                               (hipStream_t)stream, *s, energy, all_agents, changed_prefix,
-                               changed_states);
-        }
+        return with_energy_layout<H>(s->map_w, LaunchFlagged<H>{s, energy, all_agents, changed_prefix, changed_states,
+                                                               (hipStream_t)stream});
     });
-    return launch_status();
+    return JL_ERR_PROFILE;
 }
 
 extern "C" int jl_goal_changed_refresh(const jl_sim_t* s, uint8_t* energy, int64_t* prefix, int64_t* count,
@@ -317,12 +390,14 @@ extern "C" int jl_goal_changed_refresh(const jl_sim_t* s, uint8_t* energy, int64
     if (changed_states && (!s->cur_x || !s->cur_y || !s->actions)) return JL_ERR_ARG;
     const int64_t N = (int64_t)s->n_envs * s->n_agents;
     const int cells = s->map_w * s->map_h;
-    if (N <= (int64_t)kRefreshThreads * kRefreshGroups && s->map_w <= kWave && cells <= 4096) {
+    // (rows of 256 columns: 16 wavefronts of that search would not fit the
+    // registers)
+    if (N <= (int64_t)kRefreshThreads * kRefreshGroups && s->map_w <= kWave && cells <= 4096 && s->map_h < 256) {
         const unsigned grid = (unsigned)((N + kRefreshThreads - 1) / kRefreshThreads);
-        const size_t lds = (size_t)kRefreshWaves * cells;
         JL_DISPATCH_H(s->map_h, {
-            hipLaunchKernelGGL(goal_changed_refresh_kernel<H>, dim3(grid), dim3(kRefreshThreads), lds,
-                               (hipStream_t)stream, *s, energy, prefix, count, changed_states);
+            if constexpr (H < 256)
+                hipLaunchKernelGGL(goal_changed_refresh_kernel<H>, dim3(grid), dim3(kRefreshThreads), 0,
+                                   (hipStream_t)stream, *s, energy, prefix, count, changed_states);
         });
         return launch_status();
     }
