@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/jointloom.h"
 
 namespace jl {
@@ -102,13 +104,18 @@ __device__ __forceinline__ uint32_t byte_sum(uint32_t w) {
     return (w & 0xFFu) + ((w >> 8) & 0xFFu) + ((w >> 16) & 0xFFu) + (w >> 24);
 }
 
-// Compute units of the current device (grids of looping kernels are sized to them).
+// Compute units of the current device (grids of looping kernels are sized to
+// them); looked up once per device.
 inline int device_cus() {
+    static std::atomic<int> known[64];
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 256;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    const bool slot = dev >= 0 && dev < 64;
+    if (slot && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         return 256;
-    return cus > 0 ? cus : 256;
+    if (slot) known[dev].store(cus, std::memory_order_relaxed);
+    return cus;
 }
 
 // Map-profile dispatch on the column count H (a compile-time divisor).

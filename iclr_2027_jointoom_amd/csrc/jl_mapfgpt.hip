@@ -1389,7 +1389,7 @@ __host__ __device__ inline BuildLayout build_layout(int A, int W, int H, int wav
     return L;
 }
 
-// Workgroup size of the single-launch build: one thread per agent.
+// Smallest workgroup of the single-launch build: one thread per agent.
 __host__ __device__ inline int build_threads(int A) { return A <= 512 ? 512 : 1024; }
 
 // Lowest agent id keeps a shared cell of the uint16 map: min of the 16-bit
@@ -2022,10 +2022,24 @@ bool single_launch(const jl_mapfgpt_t* b) {
     return build_layout(b->n_agents, b->map_w, b->map_h, threads / kWave).total <= 160 * 1024;
 }
 
+// Workgroup size of a single-launch build: build_threads, or 1,024 threads
+// for envs of at most 512 agents too while two such workgroups per CU hold
+// every env (and their LDS and the env's egos allow it).  An env's egos and
+// changed fields then run on twice the wavefronts, which a batch of few envs
+// leaves idle otherwise: 1 env of 64 agents 10.9 -> 9.1 us; 512 envs of 100
+// agents, 16 of which search all their fields anew, 210 -> 197 us.  With more envs than that,
+// four workgroups of 512 threads per CU run in one round where two of 1,024
+// would take two.
+int launch_threads(const jl_mapfgpt_t* b) {
+    const int threads = build_threads(b->n_agents);
+    const bool few = b->n_envs <= 2 * device_cus() && b->n_agents > 2 * (threads / kWave);
+    return few && build_layout(b->n_agents, b->map_w, b->map_h, 1024 / kWave).total <= kLdsBytes / 2 ? 1024 : threads;
+}
+
 template <int H, bool kRows>
 int launch_single(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx, const int16_t* cy,
                   const int16_t* gx, const int16_t* gy, hipStream_t stream) {
-    const int threads = build_threads(b->n_agents);
+    const int threads = launch_threads(b);
     const size_t lds = build_layout(b->n_agents, b->map_w, H, threads / kWave).total;
     const dim3 grid(b->n_envs);
 #define JL_LAUNCH_BUILD(R, T)                                                                      \
