@@ -711,12 +711,21 @@ constexpr int kTokThreads = 1024;
 // first, clears them at its start, so a healthy launch never reaches it).
 constexpr int kDiagSpinLimit = 1 << 16;
 constexpr int kTokWaves = kTokThreads / kWave;
-// Egos per workgroup of a two-launch build: every workgroup stages its whole
-// env, so a workgroup takes the whole env (in steps of 128) up to 512 egos;
-// larger envs span ceil(A / 512) workgroups, whose LDS (under 80 KB up to
-// 1024 agents on any map) lets two share a CU (a single launch takes its
-// whole env).
-__host__ __device__ inline int ego_slice(int A) { return A > 512 ? 512 : (A + 127) / 128 * 128; }
+// Egos per workgroup of a two-launch build.  Every workgroup stages its whole
+// env, so a workgroup takes the whole env up to 512 egos and larger envs span
+// ceil(A / 512) workgroups, whose LDS (under 80 KB up to 1024 agents on any
+// map) lets two share a CU (a single launch takes its whole env); where that
+// leaves CUs without their two workgroups, the slices are halved, down to one
+// pair of egos per wavefront: 48 envs of 97 agents on 96 x 96 maps 11.2 -> 8.0
+// us, 64 of 128 on 128 x 128 12.6 -> 8.6 us.
+constexpr int kMaxSlice = 512;
+constexpr int kMinSlice = 2 * kTokWaves;
+inline int ego_slice(int envs, int A) {
+    int slice = kMaxSlice;
+    while (slice > kMinSlice && (slice / 2 >= A || (int64_t)envs * ((A + slice - 1) / slice) < 2 * device_cus()))
+        slice /= 2;
+    return slice;
+}
 constexpr int kDenseCellLimit = 16384;     // map cells up to which the agent map is dense
 // A window is read as 11 rows x 3 tile columns of 16-byte tile-row segments
 // (8 cells each): the 11 columns of a row span 2 or 3 tile columns.
@@ -876,11 +885,10 @@ __device__ __forceinline__ void publish_single_diagnostics(const jl_mapfgpt_t& b
 // The token pass of a two-launch build (pass 1 has written the state rows and
 // agent info words).
 template <int H, bool kDense>
-__global__ __launch_bounds__(kTokThreads) void tokens_kernel(jl_mapfgpt_t b) {
+__global__ __launch_bounds__(kTokThreads) void tokens_kernel(jl_mapfgpt_t b, int slice) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int A = b.n_agents, W = b.map_w;
     // workgroup = (env, slice of egos); every slice stages the whole env
-    const int slice = ego_slice(A);
     const int parts = (A + slice - 1) / slice;
     const int env = blockIdx.x / parts;
     const int part = blockIdx.x - env * parts;
@@ -2097,12 +2105,12 @@ int build(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx, const i
             rc = status(hipEventRecord((hipEvent_t)b->token_events[0], stream));
             if (rc) return rc;
         }
-        const int slice = ego_slice(b->n_agents);
+        const int slice = ego_slice(b->n_envs, b->n_agents);
         const dim3 grid2((unsigned)b->n_envs * ((b->n_agents + slice - 1) / slice));
         if (L.dense) {
-            hipLaunchKernelGGL((tokens_kernel<H, true>), grid2, dim3(kTokThreads), L.total, stream, *b);
+            hipLaunchKernelGGL((tokens_kernel<H, true>), grid2, dim3(kTokThreads), L.total, stream, *b, slice);
         } else {
-            hipLaunchKernelGGL((tokens_kernel<H, false>), grid2, dim3(kTokThreads), L.total, stream, *b);
+            hipLaunchKernelGGL((tokens_kernel<H, false>), grid2, dim3(kTokThreads), L.total, stream, *b, slice);
         }
         rc = launch_status();
         if (rc) return rc;
