@@ -265,23 +265,31 @@ constexpr int kHighPlanes = kFieldPlanes - 4;
 // LDS of one wavefront's high planes: [plane][lane] 64-bit words.
 constexpr int kHighPlaneBytes = kHighPlanes * kWave * 8;
 
+// a ^ b ^ c, one three-input bit operation per half.
+__device__ __forceinline__ uint64_t xor3(uint64_t a, uint64_t b, uint64_t c) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_bitop3_b32((uint32_t)a, (uint32_t)b, (uint32_t)c, 0x96);
+    const uint32_t hi =
+        (uint32_t)__builtin_amdgcn_bitop3_b32((uint32_t)(a >> 32), (uint32_t)(b >> 32), (uint32_t)(c >> 32), 0x96);
+    return ((uint64_t)hi << 32) | lo;
+}
+
 // wave_bfs_batched without a distance array: the level of every reached cell
 // of this lane's row is left bit-sliced, bits 0-3 in lowp (lowp[b] bit y =
 // bit b of the level of cell (lane, y)) and bits 4-11 in s_high[b - 4][lane]
 // (this wavefront's kHighPlaneBytes of LDS), and the reached cells in vis
-// (the start included, at level 0).  One wavefront, one map row per lane,
-// rows of at most 64 columns.  Batch b runs levels 16 b + 1 .. 16 b + 16
-// unrolled; with a[j] the free cells not reached before batch level j, the
-// cells of level 16 b + 1 + j are a[j] ^ a[j + 1], so the low level bits of
-// the batch come from a few of those snapshots (bit 1: levels 16 b + 2, 3,
-// 6, 7, 10, 11, 14, 15 = (a1 ^ a3) | (a5 ^ a7) | (a9 ^ a11) | (a13 ^ a15);
-// bit 2: (a3 ^ a7) | (a11 ^ a15); bit 3: a7 ^ a15), the high bits are b for
-// a0 ^ a15 and b + 1 for a15 ^ a16 (level 16 b + 16), ORed into the LDS
-// planes by LDS atomics once per batch, and bit 0 is no work at all: a grid
-// is bipartite, so a level's parity is that of the Manhattan distance,
-// x + y + gx + gy.  Per level only the expansion and the update of the free
-// cells remain.  The search stops after the first batch whose last level
-// reached nothing (levels past the last reach nothing).
+// (the start included, at level 0); the planes of cells not reached hold
+// anything.  One wavefront, one map row per lane, rows of at most 64 columns.
+// Batch b runs levels 16 b + 1 .. 16 b + 16 unrolled.  A cell's level bits
+// follow the search until the cell is reached: whenever the level's number
+// changes a bit, that bit's plane is flipped at the cells still free (bit 1
+// after each odd level, bit 2 after every fourth, bit 3 after every eighth;
+// two flips at a time, one three-input bit operation), and once per batch the
+// planes of the batch number's changed bits, two on average, by LDS atomics
+// (ORing the batch number into every plane of its set bits took ten times
+// the VALU work).  Bit 0 is no work at all: a grid is bipartite, so a level's
+// parity is that of the Manhattan distance, x + y + gx + gy.  The search
+// stops after the first batch whose last level reached nothing (levels past
+// the last reach nothing).
 template <int H>
 __device__ void wave_bfs_levels(uint64_t fr, int gx, int gy, uint64_t& vis, uint64_t (&lowp)[4],
                                 uint64_t* s_high) {
@@ -294,37 +302,21 @@ __device__ void wave_bfs_levels(uint64_t fr, int gx, int gy, uint64_t& vis, uint
 #pragma unroll
     for (int p = 0; p < kHighPlanes; ++p) s_high[p * kWave + lane] = 0;
     for (int b = 0;; ++b) {
-        // snapshots are folded into the planes as soon as their partner
-        // exists, so that few of them are live at once
-        const uint64_t a0 = avail;
-        uint64_t s1 = 0, s3 = 0, s5 = 0, s7 = 0, s9 = 0, s11 = 0, s13 = 0, most = 0, last = 0;
+        uint64_t odd = 0, third = 0, seventh = 0;  // free cells at the first of two flips
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
+        for (int j = 1; j <= 16; ++j) {
             front = level_step(from_lane_below(front), from_lane_above(front), front << 1, front >> 1, avail);
-            switch (j + 1) {  // avail is now a[j + 1]
-                case 1: s1 = avail; break;
-                case 3: lowp[1] |= s1 ^ avail; s3 = avail; break;
-                case 5: s5 = avail; break;
-                case 7: lowp[1] |= s5 ^ avail; lowp[2] |= s3 ^ avail; s7 = avail; break;
-                case 9: s9 = avail; break;
-                case 11: lowp[1] |= s9 ^ avail; s11 = avail; break;
-                case 13: s13 = avail; break;
-                case 15:
-                    lowp[1] |= s13 ^ avail;
-                    lowp[2] |= s11 ^ avail;
-                    lowp[3] |= s7 ^ avail;
-                    most = a0 ^ avail;
-                    last = avail;
-                    break;
-                case 16: last ^= avail; break;
-                default: break;
+            if (j % 4 == 1) odd = avail;
+            if (j % 4 == 3) lowp[1] = xor3(lowp[1], odd, avail);
+            if (j % 8 == 3) third = avail;
+            if (j % 8 == 7) lowp[2] = xor3(lowp[2], third, avail);
+            if (j == 7) seventh = avail;
+            if (j == 15) {
+                lowp[3] = xor3(lowp[3], seventh, avail);
+                const int hb = __builtin_amdgcn_readfirstlane(b), change = hb ^ (hb + 1);
+                for (int k = 0; k < kHighPlanes && (change >> k); ++k)
+                    atomicXor(reinterpret_cast<unsigned long long*>(s_high + k * kWave + lane), avail);
             }
-        }
-        const int hb = __builtin_amdgcn_readfirstlane(b), hn = hb + 1;
-#pragma unroll
-        for (int k = 0; k < kHighPlanes; ++k) {
-            const uint64_t m = (((hb >> k) & 1) ? most : 0ull) | (((hn >> k) & 1) ? last : 0ull);
-            if (((hb | hn) >> k) & 1) atomicOr(reinterpret_cast<unsigned long long*>(s_high + k * kWave + lane), m);
         }
         if (!__any(front != 0)) break;
     }
@@ -342,6 +334,12 @@ __device__ __forceinline__ uint64_t transpose8x8(uint64_t x) {
     t = (x ^ (x >> 28)) & 0x00000000F0F0F0F0ull;
     x = x ^ t ^ (t << 28);
     return x;
+}
+
+// Bytes q of four words, in a word.
+__device__ __forceinline__ uint32_t gather_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t q) {
+    const uint32_t sel = 0x0C0C0400u + q * 0x0101u;
+    return __builtin_amdgcn_perm(b, a, sel) | __builtin_amdgcn_perm(d, c, sel) << 16;
 }
 
 // ---------------------------------------------------------------------------
@@ -700,12 +698,6 @@ __device__ __forceinline__ void meet_rows(LaneWords<H, R>& a, LaneWords<H, R>& b
             b[i] = v.y;
         }
     }
-}
-
-// Bytes q of four words, in a word.
-__device__ __forceinline__ uint32_t gather_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t q) {
-    const uint32_t sel = 0x0C0C0400u + q * 0x0101u;
-    return __builtin_amdgcn_perm(b, a, sel) | __builtin_amdgcn_perm(d, c, sel) << 16;
 }
 
 }  // namespace jl
