@@ -34,6 +34,14 @@ __device__ __forceinline__ uint64_t from_lane_above(uint64_t v) {
     return ((uint64_t)hi << 32) | lo;
 }
 
+__device__ __forceinline__ uint32_t word_from_below(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xF, 0xF, true);
+}
+
+__device__ __forceinline__ uint32_t word_from_above(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xF, 0xF, true);
+}
+
 // One level of a row held in 64 bits: the new frontier (the cells of `avail`
 // that neighbour the frontier: `up` / `down` its rows of the lanes below
 // and above, `left` / `right` its own row shifted by one column) is returned
@@ -265,64 +273,124 @@ constexpr int kHighPlanes = kFieldPlanes - 4;
 // LDS of one wavefront's high planes: [plane][lane] 64-bit words.
 constexpr int kHighPlaneBytes = kHighPlanes * kWave * 8;
 
-// a ^ b ^ c, one three-input bit operation per half.
-__device__ __forceinline__ uint64_t xor3(uint64_t a, uint64_t b, uint64_t c) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_bitop3_b32((uint32_t)a, (uint32_t)b, (uint32_t)c, 0x96);
-    const uint32_t hi =
-        (uint32_t)__builtin_amdgcn_bitop3_b32((uint32_t)(a >> 32), (uint32_t)(b >> 32), (uint32_t)(c >> 32), 0x96);
-    return ((uint64_t)hi << 32) | lo;
+// The even columns (y = 2 i) and the odd columns (y = 2 i + 1) of one map row
+// of at most 64 columns, bit i.
+struct ColumnPair {
+    uint32_t even, odd;
+};
+
+// A row's words (H / 32 of them) unshuffled: three delta swaps gather the
+// even and the odd bits of each 16, byte permutes do the rest.
+template <int H>
+__device__ __forceinline__ ColumnPair split_columns(uint64_t row) {
+    static_assert(H == 32 || H == 64, "one or two words per row");
+    uint32_t w[2] = {(uint32_t)row, (uint32_t)(row >> 32)};
+#pragma unroll
+    for (int k = 0; k < H / 32; ++k) {
+        uint32_t t = (w[k] ^ (w[k] >> 1)) & 0x22222222u;
+        w[k] ^= t ^ (t << 1);
+        t = (w[k] ^ (w[k] >> 2)) & 0x0C0C0C0Cu;
+        w[k] ^= t ^ (t << 2);
+        t = (w[k] ^ (w[k] >> 4)) & 0x00F000F0u;
+        w[k] ^= t ^ (t << 4);
+    }
+    if (H == 32) w[1] = 0;
+    return {__builtin_amdgcn_perm(w[1], w[0], 0x06040200u), __builtin_amdgcn_perm(w[1], w[0], 0x07050301u)};
+}
+
+// The cells of one colour of the checkerboard that are in r's cells of the
+// other colour or next to them, for wave_bfs_levels: index i of the other
+// colour is a neighbour in this row and in the rows of both adjacent lanes,
+// and so is this row's index i - 1 or i + 1, which `turn` rotates into place
+// and `keep` clears of the bit that came round.
+__device__ __forceinline__ uint32_t next_colour(uint32_t r, uint32_t turn, uint32_t keep) {
+    const uint32_t beside = __builtin_amdgcn_alignbit(r, r, turn);
+    uint32_t t = (uint32_t)__builtin_amdgcn_bitop3_b32(beside, keep, r, 0xEA);  // (beside & keep) | r
+    t |= word_from_below(r);
+    return t | word_from_above(r);
+}
+
+// a ^ b ^ c, one instruction.
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    return (uint32_t)__builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
 }
 
 // wave_bfs_batched without a distance array: the level of every reached cell
-// of this lane's row is left bit-sliced, bits 0-3 in lowp (lowp[b] bit y =
-// bit b of the level of cell (lane, y)) and bits 4-11 in s_high[b - 4][lane]
-// (this wavefront's kHighPlaneBytes of LDS), and the reached cells in vis
-// (the start included, at level 0); the planes of cells not reached hold
-// anything.  One wavefront, one map row per lane, rows of at most 64 columns.
-// Batch b runs levels 16 b + 1 .. 16 b + 16 unrolled.  A cell's level bits
-// follow the search until the cell is reached: whenever the level's number
-// changes a bit, that bit's plane is flipped at the cells still free (bit 1
-// after each odd level, bit 2 after every fourth, bit 3 after every eighth;
-// two flips at a time, one three-input bit operation), and once per batch the
-// planes of the batch number's changed bits, two on average, by LDS atomics
-// (ORing the batch number into every plane of its set bits took ten times
-// the VALU work).  Bit 0 is no work at all: a grid is bipartite, so a level's
-// parity is that of the Manhattan distance, x + y + gx + gy.  The search
-// stops after the first batch whose last level reached nothing (levels past
-// the last reach nothing).
+// of this lane's row is left bit-sliced, bits 1-3 in lowp[0..2] and bits 4-11
+// in s_high[b - 4][lane] (this wavefront's kHighPlaneBytes of LDS), the
+// reached cells in vis (the start included, at level 0; it must be a free
+// cell); the planes of cells not reached hold anything.  One wavefront, one
+// map row per lane, rows of at most 64 columns.
+//
+// A grid is bipartite: the cells at even levels are those of the start's
+// colour of the checkerboard, and a level only reaches cells of the other
+// colour than the one before.  A row's cells of the start's colour (`own`)
+// and the others (`off`) are a 32-bit word each, and a level is one step from
+// one word to the other, five VALU instructions: the words hold everything
+// reached so far, since a reached cell but the start has a reached neighbour
+// one level below it, so no frontier and no set of cells still free is kept.
+// (Both colours in one 64-bit word, twice the words at every level, and a
+// frontier beside the cells still free: ten instructions.)  Bit 0 of a level
+// is its cell's colour.  With m the level's number >> 1, a cell reached at m
+// lies outside the words of steps 0 .. m - 1, so bit 0 of m is the parity of
+// the number of steps, bit 1 of the number of odd steps, bit 2 of every
+// fourth's, at which the cell is outside its word: two steps at a time are
+// one three-input exclusive OR (the complements cancel).  Batch b runs levels
+// 16 b + 1 .. 16 b + 16 unrolled and flips, at the cells outside, the planes
+// of the batch number's changed bits, two on average, by LDS atomics.  The
+// search stops after the first batch whose last level reached nothing.
+//
+// An even column's off-colour neighbours in its row have its own index and
+// the index below, an odd column's its own and the index above.  s_high's
+// words hold own in their lower half and off in their upper half.
 template <int H>
-__device__ void wave_bfs_levels(uint64_t fr, int gx, int gy, uint64_t& vis, uint64_t (&lowp)[4],
+__device__ void wave_bfs_levels(ColumnPair free, int gx, int gy, ColumnPair& vis, ColumnPair (&lowp)[3],
                                 uint64_t* s_high) {
-    static_assert(RowWords<H>::HW == 1, "one 64-bit word per row");
     const int lane = threadIdx.x & (kWave - 1);
-    uint64_t front = lane == gx ? 1ull << gy : 0ull;
-    uint64_t avail = fr & ~front;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) lowp[p] = 0;
+    const bool own_odd = (lane + gx + gy) & 1;  // own: this row's odd columns
+    const uint32_t free_own = own_odd ? free.odd : free.even, free_off = own_odd ? free.even : free.odd;
+    const uint32_t start = lane == gx ? 1u << (gy >> 1) : 0u;
+    const uint32_t to_off = own_odd ? 31u : 1u, to_own = 32u - to_off;  // right by 1 or left by 1
+    const uint32_t keep_off = own_odd ? ~1u : ~0u >> 1, keep_own = own_odd ? ~0u >> 1 : ~1u;
+    uint32_t own = start, off = 0, last;
+    uint32_t po[3] = {0, 0, 0}, pf[3] = {0, 0, 0};
 #pragma unroll
     for (int p = 0; p < kHighPlanes; ++p) s_high[p * kWave + lane] = 0;
     for (int b = 0;; ++b) {
-        uint64_t odd = 0, third = 0, seventh = 0;  // free cells at the first of two flips
+        uint32_t so[3] = {0, 0, 0}, sf[3] = {0, 0, 0};  // the words at the first of two flips
 #pragma unroll
-        for (int j = 1; j <= 16; ++j) {
-            front = level_step(from_lane_below(front), from_lane_above(front), front << 1, front >> 1, avail);
-            if (j % 4 == 1) odd = avail;
-            if (j % 4 == 3) lowp[1] = xor3(lowp[1], odd, avail);
-            if (j % 8 == 3) third = avail;
-            if (j % 8 == 7) lowp[2] = xor3(lowp[2], third, avail);
-            if (j == 7) seventh = avail;
-            if (j == 15) {
-                lowp[3] = xor3(lowp[3], seventh, avail);
-                const int hb = __builtin_amdgcn_readfirstlane(b), change = hb ^ (hb + 1);
-                for (int k = 0; k < kHighPlanes && (change >> k); ++k)
-                    atomicXor(reinterpret_cast<unsigned long long*>(s_high + k * kWave + lane), avail);
+        for (int k = 0; k < 8; ++k) {
+            off = next_colour(own, to_off, keep_off) & free_off;
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                const int every = 1 << p;
+                if (k % (2 * every) == every - 1) {
+                    so[p] = own;
+                    sf[p] = off;
+                }
+                if (k % (2 * every) == 2 * every - 1) {
+                    po[p] = xor3(po[p], so[p], own);
+                    pf[p] = xor3(pf[p], sf[p], off);
+                }
             }
+            if (k == 7) {
+                const int hb = __builtin_amdgcn_readfirstlane(b), change = hb ^ (hb + 1);
+                const uint64_t outside = ~((uint64_t)off << 32 | own);
+                for (int p = 0; p < kHighPlanes && (change >> p); ++p)
+                    atomicXor(reinterpret_cast<unsigned long long*>(s_high + p * kWave + lane), outside);
+            }
+            last = own;
+            own = (uint32_t)__builtin_amdgcn_bitop3_b32(next_colour(off, to_own, keep_own), free_own, start, 0xEA);
         }
-        if (!__any(front != 0)) break;
+        if (!__any(own != last)) break;
     }
-    vis = fr & ~avail;
-    const uint64_t odd_cols = ((lane + gx + gy) & 1) ? 0x5555555555555555ull : 0xAAAAAAAAAAAAAAAAull;
-    lowp[0] = vis & odd_cols;
+    vis.even = own_odd ? off : own;
+    vis.odd = own_odd ? own : off;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        lowp[p].even = own_odd ? pf[p] : po[p];
+        lowp[p].odd = own_odd ? po[p] : pf[p];
+    }
 }
 
 // 8x8 bit-matrix transpose: bit c of byte b moves to bit b of byte c.
@@ -368,14 +436,6 @@ __device__ __forceinline__ uint32_t gather_bytes(uint32_t a, uint32_t b, uint32_
 // A wavefront none of whose rows, overlap included, holds a frontier cell
 // leaves those 8 levels out.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t word_from_below(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xF, 0xF, true);
-}
-
-__device__ __forceinline__ uint32_t word_from_above(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xF, 0xF, true);
-}
-
 constexpr int kSplitLevels = 8;  // levels between two exchanges of a split search
 
 template <int H, int R>

@@ -207,20 +207,23 @@ __device__ void store_field_tiles(const jl_mapfgpt_t& b, size_t agent_index, con
 
 // refresh_field on a marked map of at most 64 rows of at most 64 columns,
 // with no LDS field: wave_bfs_levels leaves every reached cell's level in
-// bit planes (the high ones in s_high, this wavefront's kHighPlaneBytes of
-// LDS); the greedy marks come from the two low planes without any
-// comparison of distances (two reachable neighbours' levels differ by
-// exactly one, the grid being bipartite, so a reachable neighbour is closer
-// iff a0 ^ a1 ^ b1, with a0, a1 the cell's level bits 0-1 and b1 the
-// neighbour's bit 1); and each lane turns its map row into the field's
-// 8-cell tile-row segments, two 8x8 bit transposes per segment (level bits
-// 0-7, then level bits 8-11 and the four mark bits), stored as 16-byte words
-// (consecutive lanes, consecutive rows of a strip).  Same tiles and info
-// bits as refresh_field (no level of such a map can overflow the frontier).
+// bit planes, the even and the odd columns of a row apart (the high planes in
+// s_high, this wavefront's kHighPlaneBytes of LDS); the greedy marks come
+// from the two low planes without any comparison of distances (two reachable
+// neighbours' levels differ by exactly one, the grid being bipartite, so a
+// reachable neighbour is closer iff a0 ^ a1 ^ b1, with a0, a1 the cell's
+// level bits 0-1 and b1 the neighbour's bit 1); and each lane turns 16
+// columns at a time into two of the field's 8-cell tile-row segments, two
+// 8x8 bit transposes for the even and two for the odd columns (level bits
+// 0-7, then level bits 8-11 and the four mark bits) and byte permutes that
+// put the columns side by side, stored as 16-byte words (consecutive lanes,
+// consecutive rows of a strip).  Same tiles and info bits as refresh_field
+// (no level of such a map can overflow the frontier).
 // Bound by VALU issue when every field is new: 131,072 fields of 64 x 64
-// mazes 1.94 -> 1.68 ms, of i.i.d. maps 0.56 -> 0.50 ms, with the levels'
-// planes flipped instead of ORed (wave_bfs_levels) and a segment's bytes
-// gathered by byte permutes (about 60 VALU instructions instead of 130).  Every lane calls it with wavefront-uniform arguments.
+// mazes in 1.94 ms with the planes ORed level by level, 1.68 ms with them
+// flipped, 1.06 ms with five instead of ten instructions a level
+// (wave_bfs_levels).
+// Every lane calls it with wavefront-uniform arguments.
 template <int H>
 __device__ uint32_t refresh_field_levels(const jl_mapfgpt_t& b, size_t agent_index, uint32_t e, int gx, int gy,
                                          int spx, int spy, uint64_t* s_high) {
@@ -230,70 +233,95 @@ __device__ uint32_t refresh_field_levels(const jl_mapfgpt_t& b, size_t agent_ind
     bool ok = e < (uint32_t)b.n_envs && (uint32_t)gx < (uint32_t)W && (uint32_t)gy < (uint32_t)H;
     const uint32_t* env_bits = b.grid_bits + (size_t)(ok ? e : 0) * words;
     if (ok && bit_at(env_bits, gx * H + gy)) ok = false;
-    uint64_t vis = 0, pl[4] = {0, 0, 0, 0};
+    ColumnPair vis = {0, 0}, pl[3] = {};
     if (ok) {
         uint64_t fr[1][1];
         load_free_rows<H, 1>(env_bits, W, fr);
-        wave_bfs_levels<H>(fr[0][0], gx, gy, vis, pl, s_high);
+        wave_bfs_levels<H>(split_columns<H>(fr[0][0]), gx, gy, vis, pl, s_high);
     } else {
 #pragma unroll
         for (int p = 0; p < kHighPlanes; ++p) s_high[p * kWave + x] = 0;
     }
-    // neighbours' reached cells aligned with this row's columns (off the
-    // map: none), and the closer reachable neighbours
-    const uint64_t v_up = from_lane_below(vis), v_dn = from_lane_above(vis);
-    const uint64_t v_lf = vis << 1, v_rt = vis >> 1;
-    const uint64_t a01 = pl[0] ^ pl[1];
-    const uint64_t m_up = vis & v_up & (a01 ^ from_lane_below(pl[1]));
-    const uint64_t m_dn = vis & v_dn & (a01 ^ from_lane_above(pl[1]));
-    const uint64_t m_lf = vis & v_lf & (a01 ^ (pl[1] << 1));
-    const uint64_t m_rt = vis & v_rt & (a01 ^ (pl[1] >> 1));
+    // level bit 0: set in the columns that are not of the goal's colour
+    const bool own_odd = (x + gx + gy) & 1;
+    const uint32_t even0 = own_odd ? ~0u : 0u, odd0 = ~even0;
+    // per direction the neighbours' reached cells aligned with these columns
+    // (off the map: none) and, of the reachable ones, the closer.  An even
+    // column's left neighbour is the odd column of the index below, its right
+    // one that of its own index; an odd column's left neighbour is the even
+    // column of its own index, its right one that of the index above.
+    const ColumnPair q = pl[0];
+    const ColumnPair v_up = {word_from_below(vis.even), word_from_below(vis.odd)};
+    const ColumnPair v_dn = {word_from_above(vis.even), word_from_above(vis.odd)};
+    const ColumnPair v_lf = {vis.odd << 1, vis.even}, v_rt = {vis.odd, vis.even >> 1};
+    const uint32_t even01 = even0 ^ q.even, odd01 = odd0 ^ q.odd;
+    const ColumnPair m_up = {vis.even & v_up.even & (even01 ^ word_from_below(q.even)),
+                             vis.odd & v_up.odd & (odd01 ^ word_from_below(q.odd))};
+    const ColumnPair m_dn = {vis.even & v_dn.even & (even01 ^ word_from_above(q.even)),
+                             vis.odd & v_dn.odd & (odd01 ^ word_from_above(q.odd))};
+    const ColumnPair m_lf = {vis.even & v_lf.even & (even01 ^ (q.odd << 1)), vis.odd & v_lf.odd & (odd01 ^ q.even)};
+    const ColumnPair m_rt = {vis.even & v_rt.even & (even01 ^ q.odd), vis.odd & v_rt.odd & (odd01 ^ (q.even >> 1))};
     uint32_t info = ok ? 0u : kInfoBadGoal;
     if ((uint32_t)spx < (uint32_t)W && (uint32_t)spy < (uint32_t)H) {
         // greedy_mask at (spx, spy): a reachable cell's closer neighbours;
         // an unreachable one is farther than each reachable neighbour
-        const bool reached = (lane_value(vis, spx) >> spy) & 1;
-        const uint64_t q0 = lane_value(reached ? m_up : v_up, spx), q1 = lane_value(reached ? m_dn : v_dn, spx);
-        const uint64_t q2 = lane_value(reached ? m_lf : v_lf, spx), q3 = lane_value(reached ? m_rt : v_rt, spx);
-        info |= (uint32_t)((q0 >> spy) & 1) << 3 | (uint32_t)((q1 >> spy) & 1) << 2 |
-                (uint32_t)((q2 >> spy) & 1) << 1 | (uint32_t)((q3 >> spy) & 1);
+        const uint32_t odd = spy & 1 ? ~0u : 0u;
+        const auto word = [spx, odd](uint32_t of_even, uint32_t of_odd) {  // its columns' word
+            return (uint32_t)__builtin_amdgcn_readlane((int)((of_even & ~odd) | (of_odd & odd)), spx);
+        };
+        const uint32_t none = ~word(vis.even, vis.odd);
+        const uint32_t q0 = word(m_up.even, m_up.odd) | (none & word(v_up.even, v_up.odd));
+        const uint32_t q1 = word(m_dn.even, m_dn.odd) | (none & word(v_dn.even, v_dn.odd));
+        const uint32_t q2 = word(m_lf.even, m_lf.odd) | (none & word(v_lf.even, v_lf.odd));
+        const uint32_t q3 = word(m_rt.even, m_rt.odd) | (none & word(v_rt.even, v_rt.odd));
+        const int i = spy >> 1;
+        info |= (q0 >> i & 1u) << 3 | (q1 >> i & 1u) << 2 | (q2 >> i & 1u) << 1 | (q3 >> i & 1u);
     }
     // the 16 bits of every cell's tile value: level bits 0-11, then the
     // marks (bit 12 right, 13 left, 14 down, 15 up); every bit of an
     // unreachable cell set (its byte of ~vis ORed into all 16)
     if (x < (W + 7) / 8 * 8) {
-        uint4* tout = reinterpret_cast<uint4*>(b.cost_tiles + agent_index * tiled_cells(W, H));
+        uint4* out = reinterpret_cast<uint4*>(b.cost_tiles + agent_index * tiled_cells(W, H)) + x + 8;
         const int strip_words = (int)(strip_cells(W) / 8u);
-        const uint32_t* s_high32 = reinterpret_cast<const uint32_t*>(s_high);
-#pragma unroll
-        for (int half = 0; half < H / 32; ++half) {
-            // columns 32 half ..: this 32-bit half of every plane (one half
-            // after the other: the planes of both would spill)
-            asm volatile("" ::: "memory");
-            const int sh = 32 * half;
-            uint32_t hp[kHighPlanes];
-#pragma unroll
-            for (int p = 0; p < kHighPlanes; ++p) hp[p] = s_high32[(p * kWave + x) * 2 + half];
-            const uint32_t none = (uint32_t)(~vis >> sh);
-            const uint32_t p0 = (uint32_t)(pl[0] >> sh), p1 = (uint32_t)(pl[1] >> sh), p2 = (uint32_t)(pl[2] >> sh),
-                           p3 = (uint32_t)(pl[3] >> sh);
-            const uint32_t rt = (uint32_t)(m_rt >> sh), lf = (uint32_t)(m_lf >> sh), dn = (uint32_t)(m_dn >> sh),
-                           up = (uint32_t)(m_up >> sh);
-            uint4* out = tout + (4 * half + 1) * strip_words + x + 8;
+        const uint32_t* high_even = reinterpret_cast<const uint32_t*>(s_high) + 2 * x + (own_odd ? 1 : 0);
+        const uint32_t* high_odd = reinterpret_cast<const uint32_t*>(s_high) + 2 * x + (own_odd ? 0 : 1);
 #pragma unroll 1
-            for (uint32_t q = 0; q < 4; ++q) {  // segment: 8 columns
-                const uint32_t unr = __builtin_amdgcn_perm(none, none, q * 0x01010101u);
-                const uint32_t l0 = gather_bytes(p0, p1, p2, p3, q) | unr;
-                const uint32_t l1 = gather_bytes(hp[0], hp[1], hp[2], hp[3], q) | unr;
-                const uint32_t h0 = gather_bytes(hp[4], hp[5], hp[6], hp[7], q) | unr;
-                const uint32_t h1 = gather_bytes(rt, lf, dn, up, q) | unr;
+        for (uint32_t s = 0; s < H / 16; ++s) {  // two segments: 16 columns
+            // (the high planes are read again for each: kept, they would spill)
+            asm volatile("" ::: "memory");
+            // cells c = 0 .. 7 of every other column, values of two per word
+            const auto cells = [s](uint32_t reached, uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3,
+                                   const uint32_t* high, uint32_t rt, uint32_t lf, uint32_t dn, uint32_t up,
+                                   uint32_t (&v)[4]) {
+                uint32_t hp[kHighPlanes];
+#pragma unroll
+                for (int p = 0; p < kHighPlanes; ++p) hp[p] = high[p * kWave * 2];
+                const uint32_t unr = __builtin_amdgcn_perm(~reached, ~reached, s * 0x01010101u);
+                const uint32_t l0 = gather_bytes(p0, p1, p2, p3, s) | unr;
+                const uint32_t l1 = gather_bytes(hp[0], hp[1], hp[2], hp[3], s) | unr;
+                const uint32_t h0 = gather_bytes(hp[4], hp[5], hp[6], hp[7], s) | unr;
+                const uint32_t h1 = gather_bytes(rt, lf, dn, up, s) | unr;
                 const uint64_t lo = transpose8x8((uint64_t)l1 << 32 | l0);  // byte c: bits 0-7 of cell c
                 const uint64_t hi = transpose8x8((uint64_t)h1 << 32 | h0);  // byte c: bits 8-15
                 const uint32_t lo0 = (uint32_t)lo, lo1 = (uint32_t)(lo >> 32), hi0 = (uint32_t)hi, hi1 = (uint32_t)(hi >> 32);
-                out[q * strip_words] =
-                    make_uint4(__builtin_amdgcn_perm(hi0, lo0, 0x05010400u), __builtin_amdgcn_perm(hi0, lo0, 0x07030602u),
-                               __builtin_amdgcn_perm(hi1, lo1, 0x05010400u), __builtin_amdgcn_perm(hi1, lo1, 0x07030602u));
+                v[0] = __builtin_amdgcn_perm(hi0, lo0, 0x05010400u);
+                v[1] = __builtin_amdgcn_perm(hi0, lo0, 0x07030602u);
+                v[2] = __builtin_amdgcn_perm(hi1, lo1, 0x05010400u);
+                v[3] = __builtin_amdgcn_perm(hi1, lo1, 0x07030602u);
+            };
+            uint32_t ev[4], od[4];
+            cells(vis.even, even0, pl[0].even, pl[1].even, pl[2].even, high_even, m_rt.even, m_lf.even, m_dn.even,
+                  m_up.even, ev);
+            cells(vis.odd, odd0, pl[0].odd, pl[1].odd, pl[2].odd, high_odd, m_rt.odd, m_lf.odd, m_dn.odd, m_up.odd,
+                  od);
+            uint32_t w[8];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                w[2 * k] = __builtin_amdgcn_perm(od[k], ev[k], 0x05040100u);
+                w[2 * k + 1] = __builtin_amdgcn_perm(od[k], ev[k], 0x07060302u);
             }
+            out[(2 * s + 1) * strip_words] = make_uint4(w[0], w[1], w[2], w[3]);
+            out[(2 * s + 2) * strip_words] = make_uint4(w[4], w[5], w[6], w[7]);
         }
     }
     return info;
