@@ -412,19 +412,30 @@ __device__ __forceinline__ uint32_t gather_bytes(uint32_t a, uint32_t b, uint32_
 
 // ---------------------------------------------------------------------------
 // Row search: one field on a map whose rows do not fit one 64-bit word per
-// lane.  A lane holds R consecutive map rows (x = row0 + R * lane + r) as
-// H / 32 words each, so a row's x +- 1 neighbours are another register of
-// the lane or, at the ends of its block, one DPP lane move: no word of the
-// search leaves the registers.  A level costs six VALU instructions per word
-// (two funnel shifts, two ORs, two three-input bit operations).
-// Levels are held bit-sliced: bit 0 is the parity of the Manhattan offset from
-// the goal, as in wave_bfs_levels; a cell's other bits follow the search
-// until the cell is reached, which freezes them: whenever a level's number
-// changes a bit, that bit's plane is flipped at every cell still free (bit 1
-// after each odd level, bit 2 after every fourth, ...).  Bits 1-3 and kHigh
-// more are planes in registers; the planes of higher bits, flipped rarely
-// (bit k once in 2^k levels), lie in the memory of the field being searched,
-// which the caller writes last (TallPlanes).
+// lane.  A lane holds R consecutive map rows (x = row0 + R * lane + r), so a
+// row's x +- 1 neighbours are another register of the lane or, at the ends of
+// its block, one DPP lane move: no word of the search leaves the registers.
+//
+// The two colours of the checkerboard are searched in turn, as in
+// wave_bfs_levels: words of everything reached so far of the goal's colour
+// (`own`) and of the other (`off`), and a level is one step from one to the
+// other.  A row is folded in the middle: index y < H / 2 stands for the
+// columns y and H - 1 - y, which are of different colours, so an `own` word
+// holds one of the two at each index and the `off` word the other.  Whatever
+// the row's parity, the neighbours of index y are the indices y - 1 and y + 1
+// of the row itself and y of the rows beside it, and at the last index also
+// itself (the two middle columns).  A level costs five VALU instructions per
+// folded word (two funnel shifts, two ORs, one three-input bit operation),
+// half a row's words (rounded up) instead of all of them with six.
+//
+// Levels are held bit-sliced: bit 0 is the cell's colour; a cell's other bits
+// follow the search until the cell is reached, which freezes them: whenever
+// a level's number changes a bit, that bit's plane is flipped at every cell
+// not reached (bit 1 after every step of a colour, bit 2 after every second,
+// ...; two flips of bit 1 at a time).  Bits 1-3 and kHigh more are planes in
+// registers; the planes of higher bits, flipped rarely (bit k once in 2^k
+// levels), lie in the memory of the field being searched, which the caller
+// writes last (TallPlanes).  The search's result is unfolded.
 //
 // Split (kSplit): maps of more rows than one wavefront's 64 R are split over
 // the wavefronts of a workgroup.  Neighbouring wavefronts overlap: each also
@@ -433,8 +444,8 @@ __device__ __forceinline__ uint32_t gather_bytes(uint32_t a, uint32_t b, uint32_
 // owners' rows replace the overlap through LDS.  One barrier in 8 levels,
 // against one per level with the boundary rows alone (256 x 256: five
 // wavefronts instead of four, but 8 times fewer barriers and LDS round trips).
-// A wavefront none of whose rows, overlap included, holds a frontier cell
-// leaves those 8 levels out.
+// A wavefront in none of whose rows, overlap included, the first of those 8
+// levels reaches a cell leaves the others out.
 // ---------------------------------------------------------------------------
 constexpr int kSplitLevels = 8;  // levels between two exchanges of a split search
 
@@ -442,6 +453,8 @@ template <int H, int R>
 struct SearchShape {
     static constexpr int HW = H / 32;              // words per row
     static constexpr int N = R * HW;               // words per lane
+    static constexpr int M = (HW + 1) / 2;         // words per folded row and colour
+    static constexpr int K = R * M;                // words per lane and colour
     static constexpr int kGhost = kSplitLevels / R;  // overlapping lanes on each side of a split
     static constexpr int kStep = (kWave - 2 * kGhost) * R;  // rows from one wavefront of a split to the next
     static constexpr int kMaxWaves = (256 - kWave * R + kStep - 1) / kStep + 1;
@@ -467,9 +480,9 @@ __host__ __device__ constexpr int level_bits(int cells) {
 template <int H, int R, bool kSplit, bool kCount, int kWaves>
 struct SearchLds {
     using S = SearchShape<H, R>;
-    uint2 edge[kSplit ? 2 : 1][kSplit ? kWaves : 1][2][kSplit ? S::N : 1][S::kGhost];  // a split's frontier and free rows
-    uint32_t before[kCount ? kWaves : 1][kCount ? S::N * kWave : 1];                   // free cells before a batch
-    uint32_t flag[2][kWaves];                                                          // count << 1 | frontier left
+    uint2 edge[kSplit ? 2 : 1][kSplit ? kWaves : 1][2][kSplit ? S::N : 1][S::kGhost];  // a split's overlapping rows
+    uint2 before[kCount ? kWaves : 1][kCount ? S::K * kWave : 1];                      // cells reached before a batch
+    uint32_t flag[2][kWaves];                                                          // count << 1 | cells left to expand
     uint32_t count[16];
     uint32_t cell[8];
 };
@@ -489,42 +502,84 @@ struct SearchPlanes {
 template <int H, int R>
 using LaneWords = uint32_t[SearchShape<H, R>::N];
 
-// One level: the frontier's free neighbours become the frontier.
+// One lane's words of one colour.
 template <int H, int R>
-__device__ __forceinline__ void expand_rows(LaneWords<H, R>& f, LaneWords<H, R>& av) {
-    constexpr int HW = SearchShape<H, R>::HW, N = SearchShape<H, R>::N;
-    uint32_t n[N];
+using ColourWords = uint32_t[SearchShape<H, R>::K];
+
+// Index bits of row r that stand for the columns of the lower half in the own
+// words (even0: this lane's row 0 has even columns of the goal's colour).
+__device__ __forceinline__ uint32_t own_lower(bool even0, int r) {
+    return even0 == (r % 2 == 0) ? 0x55555555u : 0xAAAAAAAAu;
+}
+
+template <int H, int R>
+__device__ __forceinline__ void fold_rows(const LaneWords<H, R>& w, bool even0, ColourWords<H, R>& own,
+                                          ColourWords<H, R>& off) {
+    using S = SearchShape<H, R>;
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const int r = i / HW, k = i % HW;
-        const uint32_t up = r > 0 ? f[r > 0 ? i - HW : 0] : word_from_below(f[(R - 1) * HW + k]);
-        const uint32_t down = r + 1 < R ? f[r + 1 < R ? i + HW : 0] : word_from_above(f[k]);
-        const uint32_t left = k > 0 ? __builtin_amdgcn_alignbit(f[i], f[k > 0 ? i - 1 : 0], 31) : f[i] << 1;
-        const uint32_t right = k + 1 < HW ? __builtin_amdgcn_alignbit(f[k + 1 < HW ? i + 1 : 0], f[i], 1) : f[i] >> 1;
-        const uint32_t a = up | right, b = down | left;
-        n[i] = (uint32_t)__builtin_amdgcn_bitop3_b32(a, b, av[i], 0xA8);   // (a | b) & av
-        av[i] = (uint32_t)__builtin_amdgcn_bitop3_b32(a, b, av[i], 0x02);  // av & ~(a | b)
+    for (int i = 0; i < S::K; ++i) {
+        const int r = i / S::M, k = i % S::M;
+        const uint32_t m = own_lower(even0, r), half = S::HW % 2 != 0 && k == S::M - 1 ? 0xFFFFu : ~0u;
+        const uint32_t lower = w[r * S::HW + k], upper = __builtin_bitreverse32(w[r * S::HW + S::HW - 1 - k]);
+        own[i] = ((lower & m) | (upper & ~m)) & half;
+        off[i] = ((upper & m) | (lower & ~m)) & half;
     }
+}
+
+template <int H, int R>
+__device__ __forceinline__ void unfold_rows(const ColourWords<H, R>& own, const ColourWords<H, R>& off, bool even0,
+                                            LaneWords<H, R>& w) {
+    using S = SearchShape<H, R>;
 #pragma unroll
-    for (int i = 0; i < N; ++i) f[i] = n[i];
+    for (int i = 0; i < S::K; ++i) {
+        const int r = i / S::M, k = i % S::M;
+        const uint32_t m = own_lower(even0, r);
+        const uint32_t lower = (own[i] & m) | (off[i] & ~m), upper = (off[i] & m) | (own[i] & ~m);
+        if (S::HW % 2 != 0 && k == S::M - 1) {
+            w[r * S::HW + k] = (lower & 0xFFFFu) | __builtin_bitreverse32(upper & 0xFFFFu);
+        } else {
+            w[r * S::HW + k] = lower;
+            w[r * S::HW + S::HW - 1 - k] = __builtin_bitreverse32(upper);
+        }
+    }
+}
+
+// One level: `to` becomes the free cells of its colour beside those of `from`.
+// kPair: p is flipped at the cells outside `to` as they were and as they are;
+// kNews: returns whether `to` changed.
+template <int H, int R, bool kPair, bool kNews>
+__device__ __forceinline__ uint32_t expand_rows(const ColourWords<H, R>& from, const ColourWords<H, R>& fr,
+                                                ColourWords<H, R>& to, ColourWords<H, R>& p) {
+    using S = SearchShape<H, R>;
+    constexpr int M = S::M, K = S::K;
+    uint32_t news = 0;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const int r = i / M, k = i % M;
+        const uint32_t up = r > 0 ? from[r > 0 ? i - M : 0] : word_from_below(from[(R - 1) * M + k]);
+        const uint32_t down = r + 1 < R ? from[r + 1 < R ? i + M : 0] : word_from_above(from[k]);
+        const uint32_t before = k > 0 ? __builtin_amdgcn_alignbit(from[i], from[k > 0 ? i - 1 : 0], 31) : from[i] << 1;
+        uint32_t after;  // the last index is its own neighbour
+        if (k + 1 < M) after = __builtin_amdgcn_alignbit(from[k + 1 < M ? i + 1 : 0], from[i], 1);
+        else if (S::HW % 2 == 0) after = (uint32_t)((int32_t)from[i] >> 1);
+        else after = (from[i] >> 1) | (from[i] & 0x8000u);
+        const uint32_t a = up | after, b = down | before;
+        const uint32_t n = (uint32_t)__builtin_amdgcn_bitop3_b32(a, b, fr[i], 0xA8);  // (a | b) & fr
+        if (kPair) p[i] = xor3(p[i], to[i], n);
+        if (kNews) news |= to[i] ^ n;
+        to[i] = n;
+    }
     // levels are not interleaved: a level's words are independent enough, and
     // two levels' worth of them would not fit the registers
     __builtin_amdgcn_sched_barrier(0);
+    return news;
 }
 
-// p ^= a for every word.
+// p ^= ~a for every word.
 template <int N>
-__device__ __forceinline__ void flip_rows(uint32_t (&p)[N], const uint32_t (&a)[N]) {
+__device__ __forceinline__ void flip_outside(uint32_t (&p)[N], const uint32_t (&a)[N]) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) p[i] ^= a[i];
-}
-
-template <int N>
-__device__ __forceinline__ bool any_row(const uint32_t (&v)[N]) {
-    uint32_t o = 0;
-#pragma unroll
-    for (int i = 0; i < N; ++i) o |= v[i];
-    return o != 0;
+    for (int i = 0; i < N; ++i) p[i] = ~(p[i] ^ a[i]);
 }
 
 // Sum over the wavefront's lanes, wavefront-uniform (DPP steps that leave it in lane 63).
@@ -579,37 +634,49 @@ template <int H, int R, bool kSplit, int kHigh, int kCap, bool kCount, typename 
 __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx, int gy, int x0, int lane, int wave, int waves,
                                            Lds& s, const Tall& tall) {
     using S = SearchShape<H, R>;
-    constexpr int HW = S::HW, N = S::N, G = S::kGhost;
-    const bool own = own_lane<H, R, kSplit>(lane, wave, waves);
-    // the free cells before a batch, read back only where its levels are
+    constexpr int HW = S::HW, N = S::N, M = S::M, K = S::K, G = S::kGhost;
+    const bool mine = own_lane<H, R, kSplit>(lane, wave, waves);
+    const bool even0 = ((x0 + gx + gy) & 1) == 0;
+    // the cells reached before a batch, read back only where its levels are
     // counted (volatile: kept in LDS, not forwarded through registers)
-    volatile uint32_t* before = s.before[kCount ? wave : 0] + lane;
-    uint32_t f[N];
+    volatile uint32_t* before = reinterpret_cast<volatile uint32_t*>(s.before[kCount ? wave : 0] + lane);
+    uint32_t own[K], off[K], fr_own[K], fr_off[K];
+    uint32_t low_own[3][K], low_off[3][K], high_own[kHigh][K], high_off[kHigh][K];
     P.tall = 0;
+    {
+        uint32_t w[N];
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-        f[i] = (x0 + i / HW == gx && i % HW == (gy >> 5)) ? 1u << (gy & 31) : 0u;
-        P.avail[i] &= ~f[i];
-        P.low[0][i] = P.low[1][i] = P.low[2][i] = 0;
-#pragma unroll
-        for (int p = 0; p < kHigh; ++p) P.high[p][i] = 0;
+        for (int i = 0; i < N; ++i) {
+            w[i] = (x0 + i / HW == gx && i % HW == (gy >> 5)) ? 1u << (gy & 31) : 0u;
+            P.avail[i] |= w[i];
+        }
+        fold_rows<H, R>(P.avail, even0, fr_own, fr_off);
+        fold_rows<H, R>(w, even0, own, off);  // (the goal is in own)
     }
-    auto free_cells = [&]() -> int {
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        off[i] = 0;
+        low_own[0][i] = low_own[1][i] = low_own[2][i] = low_off[0][i] = low_off[1][i] = low_off[2][i] = 0;
+#pragma unroll
+        for (int p = 0; p < kHigh; ++p) high_own[p][i] = high_off[p][i] = 0;
+    }
+    auto reached_cells = [&]() -> int {
         int c = 0;
 #pragma unroll
-        for (int i = 0; i < N; ++i) c += __popc(P.avail[i]);
+        for (int i = 0; i < K; ++i) c += __popc(own[i]) + __popc(off[i]);
         return c;
     };
-    int slot = 0, cells = kCount ? free_cells() : 0;
+    int slot = 0, cells = kCount ? reached_cells() : 0;
     bool big = false;  // kCount: 8 levels of the batch reached more than kMaxFrontier cells
-    // After kSplitLevels levels: whether any cell is left to expand; sets
-    // big.  kSplit: the overlap is taken from its owners.
-    auto meet = [&]() -> bool {
-        const bool left = any_row(f);
+    // After kSplitLevels levels: whether any cell is left to expand (news:
+    // this lane's last level reached one); sets big.  kSplit: the overlap is
+    // taken from its owners.
+    auto meet = [&](uint32_t news) -> bool {
+        const bool left = news != 0;
         int reached = 0;
         if (kCount) {
-            const int now = free_cells();
-            reached = cells - now;
+            const int now = reached_cells();
+            reached = now > cells ? now - cells : 0;  // (a goal alone is lost)
             cells = now;
         }
         if constexpr (!kSplit) {
@@ -621,11 +688,11 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
             if (lo || hi) {
                 uint2* out = &s.edge[slot][wave][hi ? 1 : 0][0][hi ? lane - (kWave - 2 * G) : lane - G];
 #pragma unroll
-                for (int i = 0; i < N; ++i) out[i * G] = make_uint2(f[i], P.avail[i]);
+                for (int i = 0; i < K; ++i) out[i * G] = make_uint2(own[i], off[i]);
             }
-            const bool mine = __any(left && own) != 0;
-            const int sum = kCount ? wave_sum(own ? reached : 0) : 0;
-            if (lane == 0) s.flag[slot][wave] = (uint32_t)sum << 1 | (mine ? 1u : 0u);
+            const bool more = __any(left && mine) != 0;
+            const int sum = kCount ? wave_sum(mine ? reached : 0) : 0;
+            if (lane == 0) s.flag[slot][wave] = (uint32_t)sum << 1 | (more ? 1u : 0u);
             lds_barrier();
             const uint32_t all = s.flag[slot][lane < waves ? lane : 0];
             const bool from_lo = lane < G && wave > 0, from_hi = lane >= kWave - G && wave + 1 < waves;
@@ -633,10 +700,10 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
                 const uint2* in = from_lo ? &s.edge[slot][wave - 1][1][0][lane]
                                           : &s.edge[slot][wave + 1][0][0][lane - (kWave - G)];
 #pragma unroll
-                for (int i = 0; i < N; ++i) {
+                for (int i = 0; i < K; ++i) {
                     const uint2 v = in[i * G];
-                    f[i] = v.x;
-                    P.avail[i] = v.y;
+                    own[i] = v.x;
+                    off[i] = v.y;
                 }
             }
             slot ^= 1;
@@ -647,50 +714,73 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
             return __any(all & 1u) != 0;
         }
     };
+    // levels 1 .. 7 of eight, their flips included; the eighth and the flips
+    // before it follow.  False: none of them, nor the eighth, reaches a cell
+    // here (split searches), and none was searched: their flips of bits 1 and
+    // 2 cancel
+    auto seven = [&]() -> bool {
+        if (kSplit) {
+            const uint32_t news = expand_rows<H, R, false, true>(own, fr_off, off, low_off[0]);
+            if (!__any(news != 0)) return false;
+        } else {
+            expand_rows<H, R, false, false>(own, fr_off, off, low_off[0]);
+        }
+        expand_rows<H, R, true, false>(off, fr_own, own, low_own[0]);   // 2: bit 1 at steps 0 and 1
+        expand_rows<H, R, true, false>(own, fr_off, off, low_off[0]);   // 3
+        flip_outside(low_own[1], own);
+        flip_outside(low_off[1], off);
+        expand_rows<H, R, false, false>(off, fr_own, own, low_own[0]);  // 4
+        expand_rows<H, R, false, false>(own, fr_off, off, low_off[0]);  // 5
+        expand_rows<H, R, true, false>(off, fr_own, own, low_own[0]);   // 6: steps 2 and 3
+        expand_rows<H, R, true, false>(own, fr_off, off, low_off[0]);   // 7
+        flip_outside(low_own[1], own);
+        flip_outside(low_off[1], off);
+        return true;
+    };
     int overflow = 0;
     for (int b = 0;; ++b) {
         // levels 16 b + 1 .. 16 b + 16
         if (kCount) {
             big = false;
 #pragma unroll
-            for (int i = 0; i < N; ++i) before[i * kWave] = P.avail[i];
-        }
-        if (!kSplit || __any(any_row(f))) {
-#pragma unroll
-            for (int j = 1; j <= kSplitLevels; ++j) {
-                expand_rows<H, R>(f, P.avail);
-                if (j % 2 == 1) flip_rows(P.low[0], P.avail);
-                if (j % 4 == 3) flip_rows(P.low[1], P.avail);
-                if (j == 7) flip_rows(P.low[2], P.avail);
+            for (int i = 0; i < K; ++i) {
+                before[2 * i * kWave] = own[i];
+                before[2 * i * kWave + 1] = off[i];
             }
-        } else {
-            flip_rows(P.low[2], P.avail);  // (the even numbers of flips of bits 1 and 2 cancel)
         }
-        bool more = meet();
+        uint32_t news = 0;
+        bool act = seven();
+        flip_outside(low_own[2], own);
+        flip_outside(low_off[2], off);
+        if (act) news = expand_rows<H, R, false, true>(off, fr_own, own, low_own[0]);
+        bool more = meet(news);
         if (more) {
-            const bool act = !kSplit || __any(any_row(f));
-            if (act) {
-#pragma unroll
-                for (int j = 9; j < 2 * kSplitLevels; ++j) {
-                    expand_rows<H, R>(f, P.avail);
-                    if (j % 2 == 1) flip_rows(P.low[0], P.avail);
-                    if (j % 4 == 3) flip_rows(P.low[1], P.avail);
-                }
-            }
+            act = seven();
             if (kCap && b + 1 == kCap) break;  // level 16 * kCap stays out
             // the level's number reaches 16 (b + 1)
-            flip_rows(P.low[2], P.avail);
+            flip_outside(low_own[2], own);
+            flip_outside(low_off[2], off);
             const int hb = __builtin_amdgcn_readfirstlane(b), change = hb ^ (hb + 1);
-            flip_rows(P.high[0], P.avail);
 #pragma unroll
-            for (int p = 1; p < kHigh; ++p)
-                if ((change >> p) & 1) flip_rows(P.high[p], P.avail);
-            for (int p = 0; change >> (kHigh + p); ++p) {
-                tall.flip(p, p == P.tall, P.avail);
-                if (p == P.tall) P.tall = p + 1;
+            for (int p = 0; p < kHigh; ++p) {
+                if (p == 0 || ((change >> p) & 1)) {
+                    flip_outside(high_own[p], own);
+                    flip_outside(high_off[p], off);
+                }
             }
-            if (act) expand_rows<H, R>(f, P.avail);
-            more = meet();
+            if (change >> kHigh) {
+                uint32_t outside[N];
+                unfold_rows<H, R>(own, off, even0, outside);
+#pragma unroll
+                for (int i = 0; i < N; ++i) outside[i] = ~outside[i];
+                for (int p = 0; change >> (kHigh + p); ++p) {
+                    tall.flip(p, p == P.tall, outside);
+                    if (p == P.tall) P.tall = p + 1;
+                }
+            }
+            news = 0;
+            if (act) news = expand_rows<H, R, false, true>(off, fr_own, own, low_own[0]);
+            more = meet(news);
         }
         if (kCount && big) {
             // count the cells of each of the batch's levels, told apart by
@@ -703,15 +793,16 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
             for (int v = 0; v < 16; ++v) {
                 int c = 0;
 #pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    const int x = x0 + i / HW;
-                    uint32_t m = before[i * kWave] & ~P.avail[i];
-                    m &= ((x + gx + gy + v) & 1) ? 0xAAAAAAAAu : 0x55555555u;
+                for (int i = 0; i < K; ++i) {
+                    uint32_t m = (v & 1) ? off[i] & ~before[2 * i * kWave + 1] : own[i] & ~before[2 * i * kWave];
 #pragma unroll
-                    for (int p = 0; p < 3; ++p) m &= ((v >> (p + 1)) & 1) ? P.low[p][i] : ~P.low[p][i];
+                    for (int p = 0; p < 3; ++p) {
+                        const uint32_t bit = (v & 1) ? low_off[p][i] : low_own[p][i];
+                        m &= ((v >> (p + 1)) & 1) ? bit : ~bit;
+                    }
                     c += __popc(m);
                 }
-                c = wave_sum(own ? c : 0);
+                c = wave_sum(mine ? c : 0);
                 if (kSplit) {
                     if (lane == 0) atomicAdd(&s.count[v], (uint32_t)c);
                 } else if (c > kMaxFrontier) {
@@ -729,6 +820,23 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
         }
         P.batches = b + 1;
         if (!more) break;
+    }
+    // the goal, which a search without a second cell has lost, is at level 0
+#pragma unroll
+    for (int p = 0; p < 3; ++p) unfold_rows<H, R>(low_own[p], low_off[p], even0, P.low[p]);
+#pragma unroll
+    for (int p = 0; p < kHigh; ++p) unfold_rows<H, R>(high_own[p], high_off[p], even0, P.high[p]);
+    uint32_t reached[N];
+    unfold_rows<H, R>(own, off, even0, reached);
+    unfold_rows<H, R>(fr_own, fr_off, even0, P.avail);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const uint32_t goal = (x0 + i / HW == gx && i % HW == (gy >> 5)) ? 1u << (gy & 31) : 0u;
+        P.avail[i] &= ~(reached[i] | goal);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) P.low[p][i] &= ~goal;
+#pragma unroll
+        for (int p = 0; p < kHigh; ++p) P.high[p][i] &= ~goal;
     }
     return overflow;
 }
