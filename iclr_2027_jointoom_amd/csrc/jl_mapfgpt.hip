@@ -585,13 +585,15 @@ __device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, si
 // other.  A build without a
 // changed goal is the unpack alone.
 //
-// The grid is the workgroups resident at once (field_waves_per_simd), four
-// times as many in smaller batches (launch_fields), so that a batch of new
-// fields covers the chip: ranges rounded to whole passes of the workgroup's threads left 8,192
-// new fields to 64 (128 x 128) and 32 (256 x 256) workgroups.  8,192 new
-// fields of i.i.d. 128 x 128 maps (bound by VALU issue): 15.8 ms with a workgroup of two wavefronts, a barrier
-// and a 16-plane update per level -> 0.20 ms; of 256 x 256 warehouses (about
-// 80 k VALU wavefront instructions each, 1.1 ms of issue): 79.8 -> 2.22 ms.  Without a
+// The grid is the workgroups resident at once (field_waves_per_simd), or one
+// per wavefront's worth of agents, so that a batch of new fields covers the
+// chip: ranges rounded to whole passes of the workgroup's threads left 8,192
+// new fields to 64 (128 x 128) and 32 (256 x 256) workgroups.  Bound by VALU
+// issue when every field is new.  8,192 new fields of i.i.d. 128 x 128 maps
+// (14 k VALU wavefront instructions each, 0.18 ms of issue): 15.8 ms with a
+// workgroup of two wavefronts, a barrier and a 16-plane update per level ->
+// 0.25 ms; of 256 x 256 warehouses (109 k each, 1.5 ms of issue): 79.8 ->
+// 2.85 ms (3.26 with two workgroups per CU instead of three).  Without a
 // changed goal (131,072 agents, 256 x 256): 7.2 -> 6.8 us, 8.8 with the cross
 // of five cells read for every agent instead of its own cell's mark.
 // ---------------------------------------------------------------------------
@@ -2011,18 +2013,11 @@ int launch_fields(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx,
     const int N = b->n_envs * b->n_agents;
     const int waves = kSplit ? split_waves<H, R>(b->map_w) : kFieldWaves;
     // every workgroup that is resident at once, each with a field per
-    // searching wavefront (or workgroup) at least.  Batches of at most a
-    // wavefront's worth of agents per resident workgroup are dealt out in
-    // four times as many: one pass unpacks a workgroup's agents either way,
-    // and the hardware evens out the searches' lengths and the last round:
-    // 8,192 new fields of 128 x 128 maps 211 -> 200 us, of 256 x 256 maps
-    // 2275 -> 2216 us, 4,656 kept ones unchanged (24.3 us a step).  With more
-    // agents each workgroup's unpack is worth its threads.
+    // searching wavefront (or workgroup) at least
     const int resident = device_cus() * (4 * field_waves_per_simd<kSplit>() / waves);
     const int per = kSplit ? 1 : kFieldWaves;
-    const int most = (int64_t)resident * kWave >= N ? 4 * resident : resident;
     int groups = (N + per - 1) / per;
-    if (groups > most) groups = most;
+    if (groups > resident) groups = resident;
     constexpr int kMaxList = 1024;  // 16 KB of LDS list per workgroup
     if ((N + groups - 1) / groups > kMaxList) groups = (N + kMaxList - 1) / kMaxList;
     const int per_group = ((N + groups - 1) / groups + per - 1) / per * per;

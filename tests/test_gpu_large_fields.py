@@ -103,21 +103,6 @@ def test_more_fields_than_workgroups(oracle, W, H, E, A):
     build_and_compare(oracle, grids, pos, goals, ((), change))
 
 
-@pytest.mark.parametrize("W,H,E,A", [
-    (96, 64, 25, 497),   # lone searches: more agents than four times the resident workgroups take one field each
-    (130, 160, 11, 483),  # split searches: the same
-    (72, 64, 50, 985),   # more than a wavefront's worth of agents per resident workgroup
-])
-def test_lists_longer_than_a_field_each(oracle, W, H, E, A):
-    rng = np.random.default_rng(W * H + A)
-    grids = (rng.random((E, W, H)) < 0.15).astype(np.uint8)
-    free = [np.argwhere(g == 0) for g in grids]
-    pos = np.stack([f[rng.choice(len(f), A, replace=False)] for f in free])
-    goals = np.stack([f[rng.choice(len(f), A, replace=False)] for f in free])
-    change = [((int(e), int(a)), free[int(e)][0]) for e, a in zip(rng.integers(0, E, 9), rng.integers(0, A, 9))]
-    build_and_compare(oracle, grids, pos, goals, ((), change))
-
-
 def level_of_many_cells():
     """A 256x256 map whose last level holds more than 4,096 cells: an H-tree
     of corridors (4,096 leaves, all as far from the root) with further cells
