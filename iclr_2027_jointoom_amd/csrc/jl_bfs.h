@@ -434,8 +434,8 @@ __device__ __forceinline__ uint32_t gather_bytes(uint32_t a, uint32_t b, uint32_
 // not reached (bit 1 after every step of a colour, bit 2 after every second,
 // ...; two flips of bit 1 at a time).  Bits 1-3 and kHigh more are planes in
 // registers; the planes of higher bits, flipped rarely (bit k once in 2^k
-// levels), lie in the memory of the field being searched, which the caller
-// writes last (TallPlanes).  The search's result is unfolded.
+// levels), lie in LDS (the first kTall of a split search) and in the memory of
+// the field being searched, which the caller writes last (TallPlanes).  The search's result is unfolded.
 //
 // Split (kSplit): maps of more rows than one wavefront's 64 R are split over
 // the wavefronts of a workgroup.  Neighbouring wavefronts overlap: each also
@@ -482,6 +482,8 @@ struct SearchLds {
     using S = SearchShape<H, R>;
     uint2 edge[kSplit ? 2 : 1][kSplit ? kWaves : 1][2][kSplit ? S::N : 1][S::kGhost];  // a split's overlapping rows
     uint2 before[kCount ? kWaves : 1][kCount ? S::K * kWave : 1];                      // cells reached before a batch
+    static constexpr int kTall = kSplit && kCount ? 2 : 0;                             // level planes held here
+    uint32_t tall[kTall ? kTall : 1][kTall ? kWaves : 1][kTall ? S::N : 1][kTall ? kWave : 1];
     uint32_t flag[2][kWaves];                                                          // count << 1 | cells left to expand
     uint32_t count[16];
     uint32_t cell[8];

@@ -14,9 +14,9 @@
 // changed goals: goal_changed_refresh_kernel).
 //
 // Bound by VALU issue when every field is new.  16,000 fields of i.i.d.
-// 128 x 128 maps: 6.46 -> 0.34 ms (before: one wavefront per 64 jobs, one
+// 128 x 128 maps: 6.46 -> 0.22 ms (before: one wavefront per 64 jobs, one
 // after the other, with an LDS write per cell and level); 131,072 of 64 x 64:
-// 2.00 -> 0.40 ms.
+// 2.00 -> 0.40 ms (before the search by colour).
 #include "jl_bfs.h"
 #include "jl_common.h"
 

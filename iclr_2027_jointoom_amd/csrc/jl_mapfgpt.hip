@@ -396,25 +396,41 @@ constexpr int field_high() {
     return !kSplit || N < 6 ? 3 : (N < 8 ? 2 : 1);
 }
 
-// Level planes of the bits past the register planes of a field under search, kept in the tile
-// rows that the finished field will fill: plane p of word k of map row x is
-// component p & 3 of the 16-byte row x of strip 4 k + 1 + (p >> 2).  Each
-// lane reads and writes its own rows' only.
-template <int H, int R>
+// Level planes of the bits past the register planes of a field under search:
+// the first kLds of them in LDS, the others in the tile rows that the finished
+// field will fill, where plane p of word k of map row x is component p & 3 of
+// the 16-byte row x of strip 4 k + 1 + (p >> 2).  Each lane reads and writes
+// its own rows' only.  (A split search flips its first two planes past the
+// registers' 20 times in 400 levels, the others twice: with all of them in
+// memory 8,192 new fields of 256 x 256 maps took 2.2 ms, with two in LDS 1.8;
+// both fit three workgroups per CU.)
+template <int H, int R, int kLds, int kPlaneWords>
 struct TallPlanes {
     static constexpr int HW = H / 32;
     uint4* rows;           // the field's tile rows, at this lane's first map row
     uint32_t strip_words;  // 16-byte rows per strip
     int valid;             // of this lane's R rows, those it owns on the map
+    uint32_t* lds;         // this lane's word 0 of plane 0: planes kPlaneWords apart, words kWave
+    __device__ __forceinline__ uint32_t value(int p, int i) const {
+        return p < kLds ? lds[p * kPlaneWords + i * kWave] : *word(p - kLds, i);
+    }
     __device__ __forceinline__ uint32_t* word(int p, int i) const {
         return reinterpret_cast<uint32_t*>(rows + (size_t)((i % HW) * 4 + 1 + (p >> 2)) * strip_words + i / HW) + (p & 3);
     }
     template <int N>
     __device__ __forceinline__ void flip(int p, bool first, const uint32_t (&a)[N]) const {
+        if (p < kLds) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                uint32_t* w = lds + p * kPlaneWords + i * kWave;
+                *w = first ? a[i] : *w ^ a[i];
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             if (i / HW < valid) {
-                uint32_t* w = word(p, i);
+                uint32_t* w = word(p - kLds, i);
                 *w = first ? a[i] : *w ^ a[i];
             }
         }
@@ -449,9 +465,10 @@ __device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, si
     // unreachable cells; the last tile row's rows past W hold none either)
     const bool own = own_lane<H, R, kSplit>(lane, wave, waves);
     const int x0 = row0 + lane * R, left = (W + 7) / 8 * 8 - x0;
-    const TallPlanes<H, R> tiles{
+    constexpr int kPlaneWords = sizeof(s.tall[0]) / 4;
+    const TallPlanes<H, R, Lds::kTall, kPlaneWords> tiles{
         reinterpret_cast<uint4*>(b.cost_tiles + agent_index * tiled_cells(W, H)) + x0 + 8, strip_cells(W) / 8u,
-        !own || left < 0 ? 0 : (left < R ? left : R)};
+        !own || left < 0 ? 0 : (left < R ? left : R), Lds::kTall ? &s.tall[0][wave][0][lane] : nullptr};
     SearchPlanes<H, R, kFieldHigh> P;
     uint32_t vis[N];
     int overflow = 0;
@@ -545,7 +562,7 @@ __device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, si
             for (int p = 0; p < 12; ++p) {
                 t[p] = 0;
                 if (p < kFieldHigh) t[p] = P.high[p < kFieldHigh ? p : 0][i];
-                else if (P.tall > p - kFieldHigh) t[p] = *tiles.word(p - kFieldHigh, i);
+                else if (P.tall > p - kFieldHigh) t[p] = tiles.value(p - kFieldHigh, i);
             }
             if (marks) {
                 t[8] = rt & (a01 ^ rt1);
@@ -590,10 +607,11 @@ __device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, si
 // chip: ranges rounded to whole passes of the workgroup's threads left 8,192
 // new fields to 64 (128 x 128) and 32 (256 x 256) workgroups.  Bound by VALU
 // issue when every field is new.  8,192 new fields of i.i.d. 128 x 128 maps
-// (14 k VALU wavefront instructions each, 0.18 ms of issue): 15.8 ms with a
-// workgroup of two wavefronts, a barrier and a 16-plane update per level ->
-// 0.25 ms; of 256 x 256 warehouses (109 k each, 1.5 ms of issue): 79.8 ->
-// 2.85 ms (3.26 with two workgroups per CU instead of three).  Without a
+// (issue-bound): 15.8 ms with a workgroup of two wavefronts, a barrier and a
+// 16-plane update per level -> 0.21 ms; of 256 x 256 warehouses (about 80 k
+// VALU wavefront instructions each, 1.1 ms of issue): 79.8 -> 1.8 ms.  Four
+// times as many groups in smaller ranges: 5 % and 3 % less, but a step that
+// keeps its fields took up to 18 % longer.  Without a
 // changed goal (131,072 agents, 256 x 256): 7.2 -> 6.8 us, 8.8 with the cross
 // of five cells read for every agent instead of its own cell's mark.
 // ---------------------------------------------------------------------------
