@@ -51,18 +51,13 @@ constexpr int kScratchTicket = 4;
 // unreachable cells keep.  On maps of at most 4096 cells that is every field:
 // a distance there is below 4095 (at most the number of free cells minus
 // one, and a map with every cell free has a far smaller diameter).  On larger
-// maps it is the fields whose agent_info has kInfoMarked set: those whose
-// search ended before level 4095.  Readers take the distance as
-// field_distance(v, mask) with the field's mask.  cost_to_go, the API tensor,
-// holds plain distances.
+// maps the others hold plain distances, which the field itself says
+// (plain_field below).  Readers take the distance as field_distance(v, mask)
+// with the field's mask.  cost_to_go, the API tensor, holds plain distances.
 constexpr int kMarkedCells = 4096;
-constexpr uint32_t kInfoMarked = 1u << 7;  // agent_info: the field carries marks (maps of more than kMarkedCells)
-constexpr uint32_t kMarkedMask = 0x0FFFu;
+constexpr uint32_t kInfoMarked = 1u << 7;  // agent_info, from pass 1 to the token pass: the field carries marks
+constexpr uint32_t kMarkedMask = 0x0FFFu, kPlainMask = 0xFFFFu;
 __host__ __device__ inline bool marked_fields(int W, int H) { return W * H <= kMarkedCells; }
-// Distance bits of a field with the given agent_info.
-__host__ __device__ inline uint32_t field_mask(int W, int H, uint32_t info) {
-    return marked_fields(W, H) || (info & kInfoMarked) ? kMarkedMask : 0xFFFFu;
-}
 __device__ __forceinline__ uint32_t field_distance(uint32_t v, uint32_t mask) {
     return v == kUnreachable ? v : (v & mask);
 }
@@ -87,6 +82,32 @@ __host__ __device__ inline uint32_t strip_cells(int W) { return (uint32_t)tile_g
 // Offset of cell (x, y) in a tiled field, for -8 <= x < W + 8, -8 <= y < H + 8.
 __device__ __forceinline__ uint32_t tile_offset(int x, int y, int W) {
     return (uint32_t)((y >> 3) + 1) * strip_cells(W) + (uint32_t)(x + 8) * 8u + (uint32_t)(y & 7);
+}
+
+// Whether a field of a map of more than kMarkedCells cells holds plain
+// distances: kept in the field itself, so that whoever holds the tiles can
+// read them, in its border's first cells (no window reaches their row): cell
+// 0 is 0 where the field is plain, and cell 1 of the env's first field is 0
+// once any field of the env has been, so that readers look at one line per env
+// and not at one more line per field (unpack of 131,072 kept agents on 256 x
+// 256 maps: 6.4 us, and 8.0 with each field's own cell read).  Both cells are
+// kUnreachable at allocation.  A build that searches a field may set the env's
+// cell while another workgroup reads it for a field it keeps: that field was
+// searched by an earlier launch, which set the cell already if it is plain.
+__device__ __forceinline__ size_t env_plain_cell(uint32_t i, int A, size_t tcells) {
+    return (size_t)(i - i % (uint32_t)A) * tcells + 1;
+}
+__device__ __forceinline__ bool plain_field(const uint16_t* tiles, uint32_t i, uint32_t env_cell, size_t tcells) {
+    return env_cell != kUnreachable && tiles[i * tcells] != kUnreachable;
+}
+__device__ __forceinline__ void set_plain_field(uint16_t* tiles, uint32_t i, int A, size_t tcells, bool plain) {
+    tiles[i * tcells] = plain ? 0 : kUnreachable;
+    if (plain) tiles[env_plain_cell(i, A, tcells)] = 0;
+}
+// Distance bits of field i.
+__device__ __forceinline__ uint32_t field_mask(const uint16_t* tiles, uint32_t i, int W, int H, int A, size_t tcells) {
+    return marked_fields(W, H) || !plain_field(tiles, i, tiles[env_plain_cell(i, A, tcells)], tcells) ? kMarkedMask
+                                                                                                       : kPlainMask;
 }
 
 // Map profiles: H a multiple of 32 (whole bitmap words per row, as

@@ -9,8 +9,9 @@
 //
 // Distances are read from the builder's tiled fields (8 x 8 tiles of uint16,
 // one 128-byte line each), which hold what the builder last wrote into
-// cost_to_go (plus, on small maps, greedy marks that field_distance strips):
-// an 11 x 11 window touches 4 to 9 lines instead of 11 to 22 row-major ones.  The observation runs four agents per wavefront (two
+// cost_to_go (plus greedy marks, where the field carries them, which
+// field_distance strips): an 11 x 11 window touches 4 to 9 lines instead of 11
+// to 22 row-major ones.  The observation runs four agents per wavefront (two
 // window cells per lane and agent, all loads of the four in flight together,
 // the window reductions as DPP steps); the 16 agents of a workgroup assemble
 // their floats in LDS, which leave as one contiguous run of 16-byte stores.
@@ -52,7 +53,6 @@ __device__ __forceinline__ int wave_min(int v) { return wave_reduce<false>(v); }
 // the agent's stream (best reset to -1 so the next observation re-anchors it).
 template <int H>
 __global__ __launch_bounds__(256) void reward_goals_kernel(jl_sim_t s, const uint16_t* __restrict__ tiles,
-                                                           const uint32_t* __restrict__ agent_info,
                                                            int32_t* __restrict__ best,
                                                            const int16_t* __restrict__ targets,
                                                            int length, int32_t* __restrict__ cursor,
@@ -66,8 +66,9 @@ __global__ __launch_bounds__(256) void reward_goals_kernel(jl_sim_t s, const uin
     const int b0 = best[i];
     const int k = cursor[i];
     const int xc = x < W ? x : W - 1, yc = y < H ? y : H - 1;
-    const int d = (int)field_distance(tiles[(size_t)i * tiled_cells(W, H) + tile_offset(xc, yc, W)],
-                                      field_mask(W, H, marked_fields(W, H) ? 0u : agent_info[i]));
+    const size_t tcells = tiled_cells(W, H);
+    const int d = (int)field_distance(tiles[(size_t)i * tcells + tile_offset(xc, yc, W)],
+                                      field_mask(tiles, (uint32_t)i, W, H, s.n_agents, tcells));
     rewards[i] = d < b0 ? 0.1f : 0.0f;
     int bn = min(b0, d);
     const bool hit = x == gx && y == gy;
@@ -103,7 +104,7 @@ __device__ __forceinline__ void observe_agents(const jl_sim_t& s, const jl_mapfg
     const int pxl = s.cur_x[il], pyl = s.cur_y[il];
     const int32_t bestl = best[il];
     const int resetl = b.state_packed[(size_t)il * 8 + 7];
-    const uint32_t infol = marked_fields(W, H) ? 0u : b.agent_info[il];
+    const uint32_t maskl = field_mask(b.cost_tiles, (uint32_t)il, W, H, A, tcells);
     // window cells t0 = lane, t1 = lane + 64 (a cell when < 121); t = r*11 + c
     // is (cx + r - 5, cy + c - 5)
     const int t0 = lane, t1 = lane + kWave;
@@ -136,7 +137,7 @@ __device__ __forceinline__ void observe_agents(const jl_sim_t& s, const jl_mapfg
 #pragma unroll
     for (int k = 0; k < kObsPer; ++k) {
         if (k >= nvalid) break;  // wavefront-uniform
-        const uint32_t fmask = field_mask(W, H, (uint32_t)__builtin_amdgcn_readlane((int)infol, k));
+        const uint32_t fmask = (uint32_t)__builtin_amdgcn_readlane((int)maskl, k);
         const int d0 = (in0[k] && raw0[k] != kUnreachable) ? (int)(raw0[k] & fmask) : -1;
         const int d1 = (in1[k] && raw1[k] != kUnreachable) ? (int)(raw1[k] & fmask) : -1;
         // largest reachable distance in the window (0 if none)
@@ -252,7 +253,7 @@ int check_pair(const jl_sim_t* s, const jl_mapfgpt_t* b) {
         return JL_ERR_ARG;
     if ((int64_t)s->n_envs * s->n_agents > 0x7FFFFFFF) return JL_ERR_ARG;
     if (!s->cur_x || !s->cur_y || !s->goal_x || !s->goal_y || !s->grid_ocp || !b->cost_tiles ||
-        !b->state_packed || (!marked_fields(s->map_w, s->map_h) && !b->agent_info))
+        !b->state_packed)
         return JL_ERR_ARG;
     return JL_OK;
 }
@@ -272,7 +273,7 @@ extern "C" int jl_costtracer_reward_goals(const jl_sim_t* s, const jl_mapfgpt_t*
     const int n = s->n_envs * s->n_agents;
     JL_DISPATCH_H(s->map_h, {
         hipLaunchKernelGGL((reward_goals_kernel<H>), dim3((n + 255) / 256), dim3(256), 0,
-                           (hipStream_t)stream, *s, b->cost_tiles, b->agent_info, best, targets, target_length,
+                           (hipStream_t)stream, *s, b->cost_tiles, best, targets, target_length,
                            cursor, rewards, reached, n);
     });
     return launch_status();

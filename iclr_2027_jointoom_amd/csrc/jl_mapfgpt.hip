@@ -534,6 +534,8 @@ __device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, si
     // one), from the levels' two low bits
     const bool marks = P.batches * 16 < (int)kMarkedMask;
     if (marks) info |= kInfoMarked;
+    if (lane == 0 && (!kSplit || wave == 0))
+        set_plain_field(b.cost_tiles, (uint32_t)agent_index, b.n_agents, tiled_cells(W, H), !marks);
     if (kSplit) meet_rows<H, R>(vis, P.low[0], lane, wave, waves, s);
     // the tiles: 16 bits of every cell, every bit of an unreached cell set
 #pragma unroll
@@ -635,6 +637,7 @@ __attribute__((amdgpu_waves_per_eu(field_waves_per_simd<kSplit>()))) void unpack
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int threads = waves * kWave;
+    const size_t tcells = tiled_cells(b.map_w, H);
     const int begin = blockIdx.x * per_group;
     const int end = (begin + per_group) < N ? (begin + per_group) : N;
     // the build's diagnostics start from zero; pass 2 and append_actions add
@@ -643,7 +646,7 @@ __attribute__((amdgpu_waves_per_eu(field_waves_per_simd<kSplit>()))) void unpack
     __syncthreads();
     for (int i = begin + tid; i < end; i += threads) {
         uint32_t info;
-        const uint32_t kept = b.agent_info[i] & kInfoMarked;
+        const uint32_t env_cell = b.cost_tiles[env_plain_cell((uint32_t)i, b.n_agents, tcells)];  // (in flight below)
         const uint4 st = unpack_agent<kRows>(b, i, raw_rows, cur_x, cur_y, goal_x, goal_y, info);
         const uint32_t px = st.y & 0xFFFFu, py = st.y >> 16;
         if ((st.w >> 16) != 0) {
@@ -651,8 +654,9 @@ __attribute__((amdgpu_waves_per_eu(field_waves_per_simd<kSplit>()))) void unpack
             s_list[atomicAdd(&s_n, 1)] = make_uint4((uint32_t)i, info | (st.x << 16), st.y, st.z);
             continue;
         }
-        info |= kept;
-        if (px < (uint32_t)b.map_w && py < (uint32_t)H) info |= kept_greedy<H>(b, (size_t)i, (int)px, (int)py, kept != 0);
+        const bool marked = !plain_field(b.cost_tiles, (uint32_t)i, env_cell, tcells);
+        info |= marked ? kInfoMarked : 0u;
+        if (px < (uint32_t)b.map_w && py < (uint32_t)H) info |= kept_greedy<H>(b, (size_t)i, (int)px, (int)py, marked);
         b.agent_info[i] = info;
     }
     __syncthreads();
@@ -1005,7 +1009,7 @@ __global__ __launch_bounds__(kTokThreads) void tokens_kernel(jl_mapfgpt_t b, int
             const bool third = (tyl + 2) * 8 <= ey + kRadius;
             s_seg[a] = (uint32_t)a * (uint32_t)tiled_cells(W, H) * 2u + (uint32_t)(tyl + 1) * strip_cells(W) * 2u +
                        (uint32_t)(ex - kRadius + 8) * 16u + (third ? 1u : 0u) +
-                       (field_mask(W, H, info) == kMarkedMask ? 2u : 0u);
+                       (marked_fields(W, H) || (info & kInfoMarked) ? 2u : 0u);
         }
         // the template: position (kNoAgent off the map: such an ego's row is
         // padding, and no window holds it), goal, history codes, greedy mask
@@ -1199,7 +1203,7 @@ __global__ __launch_bounds__(kTokThreads) void tokens_kernel(jl_mapfgpt_t b, int
             const int ex = (int)(pos & 0xFFFFu), ey = (int)(pos >> 16);
             // region row = dx + 5, column = dy + 5 + ((ey + 3) & 7) (see seg_load)
             const uint16_t* win = win_base + (rec.w >> 24);
-            const uint32_t fmask = (rec.z & 2u) ? kMarkedMask : 0xFFFFu;  // distance bits of the ego's field
+            const uint32_t fmask = (rec.z & 2u) ? kMarkedMask : kPlainMask;  // distance bits of the ego's field
             const uint32_t craw = win[kRadius * kRegionCols + kRadius];
             const uint32_t center = field_distance((uint32_t)__builtin_amdgcn_readfirstlane((int)craw), fmask);
             const uint32_t v0 = win[win0];  // raw tiled values: the table index strips the marks
@@ -1970,7 +1974,7 @@ __global__ __launch_bounds__(256) void cost_to_go_kernel(jl_mapfgpt_t b) {
         const size_t f = i / per_field;
         const uint32_t w = (uint32_t)(i - f * per_field);
         const uint32_t x = w / (H / 8), y8 = w - x * (H / 8);  // row, 8-cell group
-        const uint32_t fmask = field_mask(W, H, marked_fields(W, H) ? 0u : b.agent_info[f]);
+        const uint32_t fmask = field_mask(b.cost_tiles, (uint32_t)f, W, H, b.n_agents, tcells);
         v4i v = tiles[f * (tcells / 8) + (y8 + 1) * strip_words + x + 8];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -2049,8 +2053,8 @@ template <int H, int R, bool kRows>
 int launch_pass1(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx, const int16_t* cy,
                  const int16_t* gx, const int16_t* gy, hipStream_t stream) {
     const int N = b->n_envs * b->n_agents;
-    // maps whose tiled fields carry greedy marks (at most 4096 cells, 8 KB
-    // LDS fields) run pass 1 as one launch; only that launch writes marks
+    // maps of at most 4096 cells (8 KB LDS fields), whose tiled fields always
+    // carry greedy marks
     if (marked_fields(b->map_w, H)) {
         const dim3 grid((N + kWave * 4 - 1) / (kWave * 4));
         const size_t lds = (size_t)4 * marked_wave_lds(b->map_w, H);

@@ -193,18 +193,16 @@ typedef struct jl_mapfgpt {
     int32_t* tokens;            /* [N, 256] */
     uint8_t* active_mask;       /* [N] (torch.bool) */
     int32_t* diagnostics;       /* [4] overflow, bad row/action, duplicate cell, bad goal/position */
-    uint32_t* agent_info;       /* [N] workspace of this builder: greedy-move mask and
-                                   diagnostic flags of each agent, written by the first
-                                   pass of a build; bit 7, kept from build to build, says
-                                   whether the field of a map of more than 4096 cells
-                                   carries greedy marks */
+    uint32_t* agent_info;       /* [N] workspace: greedy-move mask and diagnostic flags of
+                                   each agent, written by the first pass of a build */
     uint16_t* cost_tiles;       /* [E, A, ceil(W/8) + 2, H/8 + 2, 8, 8] workspace, 0xFFFF at
                                    allocation: the same fields as cost_to_go in 8x8 tiles
                                    (one 128-byte line per tile) inside a one-tile border of
-                                   unreachable cells that no kernel writes; on maps of at
-                                   most 4096 cells, and on larger ones in the fields whose
-                                   agent_info has bit 7 set, bits 12-15 of a reachable
-                                   cell hold its greedy-move mask */
+                                   unreachable cells; on maps of at most 4096 cells, and
+                                   on larger ones in the fields whose levels all fit
+                                   bits 0-11, bits 12-15 of a reachable cell hold its
+                                   greedy-move mask (the border's first two cells, which
+                                   nothing else reads, tell those fields from the others) */
     int32_t* build_scratch;     /* [JL_BUILD_SCRATCH_WORDS] workspace, zero at construction,
                                    128-byte aligned, used with this builder's n_envs only:
                                    the single-launch build of small maps keeps in it the
