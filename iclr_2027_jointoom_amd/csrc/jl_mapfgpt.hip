@@ -766,17 +766,27 @@ constexpr int kDiagSpinLimit = 1 << 16;
 constexpr int kTokWaves = kTokThreads / kWave;
 // Egos per workgroup of a two-launch build.  Every workgroup stages its whole
 // env, so a workgroup takes the whole env up to 512 egos and larger envs span
-// ceil(A / 512) workgroups, whose LDS (under 80 KB up to 1024 agents on any
-// map) lets two share a CU (a single launch takes its whole env); where that
-// leaves CUs without their two workgroups, the slices are halved, down to one
-// pair of egos per wavefront: 48 envs of 97 agents on 96 x 96 maps 11.2 -> 8.0
-// us, 64 of 128 on 128 x 128 12.6 -> 8.6 us.
+// ceil(A / 512) workgroups (a single launch takes its whole env).  Where that
+// leaves CUs without a workgroup the slices are halved, down to one pair of
+// egos per wavefront, while every workgroup still finds a CU of its own; past
+// that, while two share a CU (their LDS, `lds` each, lets them) and have at
+// least 128 egos.  Measured (us a build that keeps its fields, by slice):
+//   96 x 96 (one workgroup's LDS per CU): 48 envs of 97 agents 128: 13.4, 64:
+//   11.8, 32 (192 workgroups): 10.5; 300 of 100 128 (300): 18.8, 64 (600):
+//   21.3; 128 of 390 512: 35.7, 256 (256): 27.0, 128 (512): 30.6;
+//   130 x 224 (two): 100 of 100 128: 15.2, 64 (200): 13.7, 32 (400): 14.6; 60
+//   of 1,000 256 (240): 29.7, 128 (480): 28.2, 64 (960): 33.8; 300 of 100 128
+//   (300): 20.0, 64 (600): 24.6.
 constexpr int kMaxSlice = 512;
 constexpr int kMinSlice = 2 * kTokWaves;
-inline int ego_slice(int envs, int A) {
+inline int ego_slice(int envs, int A, size_t lds) {
+    const int64_t alone = device_cus(), shared = 2 * lds <= kLdsBytes ? 2 * alone : alone;
+    const auto room = [&](int slice) {  // slices of this size are worth their workgroups
+        const int64_t groups = (int64_t)envs * ((A + slice - 1) / slice);
+        return groups <= alone || (groups <= shared && slice >= 128);
+    };
     int slice = kMaxSlice;
-    while (slice > kMinSlice && (slice / 2 >= A || (int64_t)envs * ((A + slice - 1) / slice) < 2 * device_cus()))
-        slice /= 2;
+    while (slice > kMinSlice && (slice / 2 >= A || room(slice / 2))) slice /= 2;
     return slice;
 }
 constexpr int kDenseCellLimit = 16384;     // map cells up to which the agent map is dense
@@ -2158,7 +2168,7 @@ int build(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx, const i
             rc = status(hipEventRecord((hipEvent_t)b->token_events[0], stream));
             if (rc) return rc;
         }
-        const int slice = ego_slice(b->n_envs, b->n_agents);
+        const int slice = ego_slice(b->n_envs, b->n_agents, L.total);
         const dim3 grid2((unsigned)b->n_envs * ((b->n_agents + slice - 1) / slice));
         if (L.dense) {
             hipLaunchKernelGGL((tokens_kernel<H, true>), grid2, dim3(kTokThreads), L.total, stream, *b, slice);

@@ -1,0 +1,38 @@
+"""The rules that choose how a call's work is cut into workgroups keep to the
+bounds that they are there for (read off the launches of a captured call)."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+LDS = 160 * 1024
+
+
+def cus():
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
+def state_build(E, A, W, H):
+    """A builder on open maps whose fields are there, its next build's launches."""
+    from iclr_2027_jointoom_amd import profile
+    from launches import launches
+
+    rng = np.random.default_rng(E + A)
+    b = profile(W, H).MapfGPTObservationBuilder(torch.zeros((E, W, H), dtype=torch.int32, device="cuda"), A)
+    st = [torch.from_numpy(rng.integers(0, n, (E, A)).astype(np.int16)).cuda() for n in (W, H, W, H)]
+    b.build_tokens_from_state(*st)
+    torch.cuda.synchronize()
+    return launches(lambda: b.build_tokens_from_state(*st))
+
+
+@pytest.mark.parametrize("W,H", [(96, 96), (130, 192)])
+@pytest.mark.parametrize("E,A", [(1, 1), (3, 600), (16, 512), (64, 128), (100, 100), (130, 128), (200, 64), (300, 100),
+                                 (150, 200), (300, 33), (600, 40)])
+def test_token_slices_run_at_once(E, A, W, H):
+    """Slices of an env's egos are cut smaller only while all of them are
+    resident at once: a second round costs what the smaller slices save."""
+    got = [k for k in state_build(E, A, W, H) if "tokens_kernel" in k.name]
+    assert len(got) == 1
+    whole = E * -(-A // 512)  # no slice cut
+    assert got[0].groups <= max(whole, cus() * min(2, LDS // got[0].lds)), got
