@@ -476,17 +476,28 @@ __host__ __device__ constexpr int level_bits(int cells) {
     return b;
 }
 
-// LDS of the searches of a workgroup of kWaves wavefronts.
+// LDS of one wavefront of a search.
+template <int H, int R, bool kSplit, bool kCount>
+struct SearchWaveLds {
+    using S = SearchShape<H, R>;
+    static constexpr int kTall = kSplit && kCount ? 2 : 0;                  // level planes held here
+    uint2 edge[kSplit ? 2 : 1][2][kSplit ? S::N : 1][kSplit ? S::kGhost : 1];  // a split's overlapping rows
+    uint2 before[kCount ? S::K * kWave : 1];                                // cells reached before a batch
+    uint32_t tall[kTall ? kTall : 1][kTall ? S::N : 1][kTall ? kWave : 1];
+};
+
+// LDS of the searches of a workgroup of at most kWaves wavefronts: a launch of
+// `waves` allocates bytes(waves).
 template <int H, int R, bool kSplit, bool kCount, int kWaves>
 struct SearchLds {
-    using S = SearchShape<H, R>;
-    uint2 edge[kSplit ? 2 : 1][kSplit ? kWaves : 1][2][kSplit ? S::N : 1][S::kGhost];  // a split's overlapping rows
-    uint2 before[kCount ? kWaves : 1][kCount ? S::K * kWave : 1];                      // cells reached before a batch
-    static constexpr int kTall = kSplit && kCount ? 2 : 0;                             // level planes held here
-    uint32_t tall[kTall ? kTall : 1][kTall ? kWaves : 1][kTall ? S::N : 1][kTall ? kWave : 1];
-    uint32_t flag[2][kWaves];                                                          // count << 1 | cells left to expand
+    using Wave = SearchWaveLds<H, R, kSplit, kCount>;
+    uint32_t flag[2][kWaves];  // count << 1 | cells left to expand
     uint32_t count[16];
     uint32_t cell[8];
+    alignas(16) Wave wave[kWaves];
+    static constexpr size_t bytes(int waves) {
+        return (sizeof(SearchLds) - (kWaves - waves) * sizeof(Wave) + 15) / 16 * 16;
+    }
 };
 
 // One wavefront's part of a search's result.
@@ -641,7 +652,14 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
     const bool even0 = ((x0 + gx + gy) & 1) == 0;
     // the cells reached before a batch, read back only where its levels are
     // counted (volatile: kept in LDS, not forwarded through registers)
-    volatile uint32_t* before = reinterpret_cast<volatile uint32_t*>(s.before[kCount ? wave : 0] + lane);
+    const auto before_words = [&]() {
+        int l = lane;
+        // the address taken afresh, or held across the search: a split of
+        // seven words per lane (224 columns) has no register left to hold it;
+        // elsewhere holding it is 1 % of a stage of new fields faster
+        if constexpr (kSplit && N == 7) asm("" : "+v"(l));
+        return reinterpret_cast<volatile uint32_t*>(s.wave[wave].before + l);
+    };
     uint32_t own[K], off[K], fr_own[K], fr_off[K];
     uint32_t low_own[3][K], low_off[3][K], high_own[kHigh][K], high_off[kHigh][K];
     P.tall = 0;
@@ -688,7 +706,7 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
         } else {
             const bool lo = lane >= G && lane < 2 * G, hi = lane >= kWave - 2 * G && lane < kWave - G;
             if (lo || hi) {
-                uint2* out = &s.edge[slot][wave][hi ? 1 : 0][0][hi ? lane - (kWave - 2 * G) : lane - G];
+                uint2* out = &s.wave[wave].edge[slot][hi ? 1 : 0][0][hi ? lane - (kWave - 2 * G) : lane - G];
 #pragma unroll
                 for (int i = 0; i < K; ++i) out[i * G] = make_uint2(own[i], off[i]);
             }
@@ -699,8 +717,8 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
             const uint32_t all = s.flag[slot][lane < waves ? lane : 0];
             const bool from_lo = lane < G && wave > 0, from_hi = lane >= kWave - G && wave + 1 < waves;
             if (from_lo || from_hi) {
-                const uint2* in = from_lo ? &s.edge[slot][wave - 1][1][0][lane]
-                                          : &s.edge[slot][wave + 1][0][0][lane - (kWave - G)];
+                const uint2* in = from_lo ? &s.wave[wave - 1].edge[slot][1][0][lane]
+                                          : &s.wave[wave + 1].edge[slot][0][0][lane - (kWave - G)];
 #pragma unroll
                 for (int i = 0; i < K; ++i) {
                     const uint2 v = in[i * G];
@@ -744,6 +762,7 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
         // levels 16 b + 1 .. 16 b + 16
         if (kCount) {
             big = false;
+            volatile uint32_t* before = before_words();
 #pragma unroll
             for (int i = 0; i < K; ++i) {
                 before[2 * i * kWave] = own[i];
@@ -792,6 +811,7 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
                 if (threadIdx.x < 16) s.count[threadIdx.x] = 0;
                 lds_barrier();
             }
+            volatile uint32_t* before = before_words();
             for (int v = 0; v < 16; ++v) {
                 int c = 0;
 #pragma unroll
@@ -853,14 +873,15 @@ __device__ __forceinline__ void meet_rows(LaneWords<H, R>& a, LaneWords<H, R>& b
     lds_barrier();  // the search's last exchange has been read
     const bool lo = lane >= G && lane < 2 * G, hi = lane >= kWave - 2 * G && lane < kWave - G;
     if (lo || hi) {
-        uint2* out = &s.edge[0][wave][hi ? 1 : 0][0][hi ? lane - (kWave - 2 * G) : lane - G];
+        uint2* out = &s.wave[wave].edge[0][hi ? 1 : 0][0][hi ? lane - (kWave - 2 * G) : lane - G];
 #pragma unroll
         for (int i = 0; i < N; ++i) out[i * G] = make_uint2(a[i], b[i]);
     }
     lds_barrier();
     const bool from_lo = lane < G && wave > 0, from_hi = lane >= kWave - G && wave + 1 < waves;
     if (from_lo || from_hi) {
-        const uint2* in = from_lo ? &s.edge[0][wave - 1][1][0][lane] : &s.edge[0][wave + 1][0][0][lane - (kWave - G)];
+        const uint2* in = from_lo ? &s.wave[wave - 1].edge[0][1][0][lane]
+                                  : &s.wave[wave + 1].edge[0][0][0][lane - (kWave - G)];
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const uint2 v = in[i * G];

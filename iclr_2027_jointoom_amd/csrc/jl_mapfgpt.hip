@@ -402,8 +402,7 @@ constexpr int field_high() {
 // the 16-byte row x of strip 4 k + 1 + (p >> 2).  Each lane reads and writes
 // its own rows' only.  (A split search flips its first two planes past the
 // registers' 20 times in 400 levels, the others twice: with all of them in
-// memory 8,192 new fields of 256 x 256 maps took 2.2 ms, with two in LDS 1.8;
-// both fit three workgroups per CU.)
+// memory 8,192 new fields of 256 x 256 maps took 2.2 ms, with two in LDS 1.8.)
 template <int H, int R, int kLds, int kPlaneWords>
 struct TallPlanes {
     static constexpr int HW = H / 32;
@@ -465,10 +464,11 @@ __device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, si
     // unreachable cells; the last tile row's rows past W hold none either)
     const bool own = own_lane<H, R, kSplit>(lane, wave, waves);
     const int x0 = row0 + lane * R, left = (W + 7) / 8 * 8 - x0;
-    constexpr int kPlaneWords = sizeof(s.tall[0]) / 4;
-    const TallPlanes<H, R, Lds::kTall, kPlaneWords> tiles{
+    using Wave = typename Lds::Wave;
+    constexpr int kPlaneWords = sizeof(Wave::tall[0]) / 4;
+    const TallPlanes<H, R, Wave::kTall, kPlaneWords> tiles{
         reinterpret_cast<uint4*>(b.cost_tiles + agent_index * tiled_cells(W, H)) + x0 + 8, strip_cells(W) / 8u,
-        !own || left < 0 ? 0 : (left < R ? left : R), Lds::kTall ? &s.tall[0][wave][0][lane] : nullptr};
+        !own || left < 0 ? 0 : (left < R ? left : R), Wave::kTall ? &s.wave[wave].tall[0][0][lane] : nullptr};
     SearchPlanes<H, R, kFieldHigh> P;
     uint32_t vis[N];
     int overflow = 0;
@@ -604,25 +604,34 @@ __device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, si
 // other.  A build without a
 // changed goal is the unpack alone.
 //
-// The grid is the workgroups resident at once (field_waves_per_simd), or one
-// per wavefront's worth of agents, so that a batch of new fields covers the
-// chip: ranges rounded to whole passes of the workgroup's threads left 8,192
+// The grid is the workgroups resident at once (field_waves_per_simd and the
+// LDS of the wavefronts that the map needs, launch_fields), or one per
+// wavefront's worth of agents, so that a batch of new fields covers the chip:
+// ranges rounded to whole passes of the workgroup's threads left 8,192
 // new fields to 64 (128 x 128) and 32 (256 x 256) workgroups.  Bound by VALU
 // issue when every field is new.  8,192 new fields of i.i.d. 128 x 128 maps
 // (issue-bound): 15.8 ms with a workgroup of two wavefronts, a barrier and a
 // 16-plane update per level -> 0.21 ms; of 256 x 256 warehouses (about 80 k
 // VALU wavefront instructions each, 1.1 ms of issue): 79.8 -> 1.8 ms.  Four
 // times as many groups in smaller ranges: 5 % and 3 % less, but a step that
-// keeps its fields took up to 18 % longer.  Without a
-// changed goal (131,072 agents, 256 x 256): 7.2 -> 6.8 us, 8.8 with the cross
-// of five cells read for every agent instead of its own cell's mark.
+// keeps its fields took longer.  With the LDS of five wavefronts whatever the
+// map needs (three workgroups per CU instead of eight, five or four): 8,192 new
+// fields of 96 x 256 maps 765 us, 128 x 256 960, 200 x 256 1,200, 100 x 160
+// 359, against 432, 785, 985 and 258.  Without a changed goal (131,072 agents,
+// 256 x 256): 6.2 us (6.7-7.2 with the workgroups of two per CU of the former
+// kernel), 8.8 with the cross of five cells read for every agent instead of
+// its own cell's mark.
 // ---------------------------------------------------------------------------
 constexpr int kFieldWaves = 4;  // wavefronts of a workgroup whose wavefronts search on their own
+constexpr size_t kFieldsStaticLds = 16;
 
 template <int H, int R, bool kSplit>
 constexpr int field_waves() {
     return kSplit ? SearchShape<H, R>::kMaxWaves : kFieldWaves;
 }
+
+template <int H, int R, bool kSplit>
+using FieldsLds = SearchLds<H, R, kSplit, true, field_waves<H, R, kSplit>()>;
 
 template <int H, int R, bool kSplit, bool kRows>
 __global__ __launch_bounds__((kWave * field_waves<H, R, kSplit>()))
@@ -630,9 +639,12 @@ __attribute__((amdgpu_waves_per_eu(field_waves_per_simd<kSplit>()))) void unpack
     jl_mapfgpt_t b, const int16_t* __restrict__ raw_rows, const int16_t* __restrict__ cur_x,
     const int16_t* __restrict__ cur_y, const int16_t* __restrict__ goal_x,
     const int16_t* __restrict__ goal_y, int per_group, int waves) {
-    __shared__ SearchLds<H, R, kSplit, true, field_waves<H, R, kSplit>()> s_search;
+    using Lds = FieldsLds<H, R, kSplit>;
     __shared__ int s_n;
-    extern __shared__ __align__(16) uint4 s_list[];  // [per_group]: agent, info | env << 16, state row words y, z
+    extern __shared__ __align__(16) uint8_t s_dynamic[];
+    Lds& s_search = *reinterpret_cast<Lds*>(s_dynamic);
+    // [per_group]: agent, info | env << 16, state row words y, z
+    uint4* s_list = reinterpret_cast<uint4*>(s_dynamic + Lds::bytes(waves));
     const int N = b.n_envs * b.n_agents;
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -2044,18 +2056,22 @@ int launch_fields(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx,
                   const int16_t* gx, const int16_t* gy, hipStream_t stream) {
     const int N = b->n_envs * b->n_agents;
     const int waves = kSplit ? split_waves<H, R>(b->map_w) : kFieldWaves;
-    // every workgroup that is resident at once, each with a field per
-    // searching wavefront (or workgroup) at least
-    const int resident = device_cus() * (4 * field_waves_per_simd<kSplit>() / waves);
-    const int per = kSplit ? 1 : kFieldWaves;
-    int groups = (N + per - 1) / per;
-    if (groups > resident) groups = resident;
+    // every workgroup that is resident at once (wavefronts per SIMD, LDS), each
+    // with a field per searching wavefront (or workgroup) at least
+    constexpr int kPer = kSplit ? 1 : kFieldWaves;
     constexpr int kMaxList = 1024;  // 16 KB of LDS list per workgroup
-    if ((N + groups - 1) / groups > kMaxList) groups = (N + kMaxList - 1) / kMaxList;
-    const int per_group = ((N + groups - 1) / groups + per - 1) / per * per;
+    int per_group = 0;
+    size_t lds = 0;
+    for (int per_cu = 4 * field_waves_per_simd<kSplit>() / waves; per_cu > 0; --per_cu) {
+        int groups = (N + kPer - 1) / kPer;
+        if (groups > device_cus() * per_cu) groups = device_cus() * per_cu;
+        if ((N + groups - 1) / groups > kMaxList) groups = (N + kMaxList - 1) / kMaxList;
+        per_group = ((N + groups - 1) / groups + kPer - 1) / kPer * kPer;
+        lds = FieldsLds<H, R, kSplit>::bytes(waves) + (size_t)per_group * sizeof(uint4);
+        if (per_cu * (lds + kFieldsStaticLds) <= kLdsBytes) break;
+    }
     hipLaunchKernelGGL((unpack_fields_kernel<H, R, kSplit, kRows>), dim3((N + per_group - 1) / per_group),
-                       dim3(kWave * waves), (size_t)per_group * sizeof(uint4), stream, *b, rows, cx, cy, gx, gy,
-                       per_group, waves);
+                       dim3(kWave * waves), lds, stream, *b, rows, cx, cy, gx, gy, per_group, waves);
     return launch_status();
 }
 

@@ -36,3 +36,15 @@ def test_token_slices_run_at_once(E, A, W, H):
     assert len(got) == 1
     whole = E * -(-A // 512)  # no slice cut
     assert got[0].groups <= max(whole, cus() * min(2, LDS // got[0].lds)), got
+
+
+@pytest.mark.parametrize("W,H", [(65, 160), (128, 192), (160, 224), (208, 224), (96, 256), (128, 256), (200, 256), (256, 256)])
+def test_split_searches_run_at_once(W, H):
+    """A map split over the wavefronts of a workgroup: the workgroups' LDS
+    leaves room for as many per CU as the launch counts on."""
+    E, A = 20, 256
+    got = [k for k in state_build(E, A, W, H) if "unpack_fields_kernel" in k.name]
+    assert len(got) == 1
+    assert got[0].groups <= cus() * (LDS // got[0].lds), got
+    # and for at least 12 of a CU's 16 wavefronts (five-wavefront groups: 15)
+    assert (LDS // got[0].lds) * got[0].threads >= 12 * 64, got
