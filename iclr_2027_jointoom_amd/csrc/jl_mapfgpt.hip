@@ -2110,23 +2110,31 @@ bool single_launch(const jl_mapfgpt_t* b) {
 }
 
 // Workgroup size of a single-launch build: build_threads, or 1,024 threads
-// for envs of at most 512 agents too while two such workgroups per CU hold
-// every env (and their LDS and the env's egos allow it).  An env's egos and
-// changed fields then run on twice the wavefronts, which a batch of few envs
-// leaves idle otherwise: 1 env of 64 agents 10.9 -> 9.1 us; 512 envs of 100
-// agents, 16 of which search all their fields anew, 210 -> 197 us.  With more envs than that,
-// four workgroups of 512 threads per CU run in one round where two of 1,024
-// would take two.
-int launch_threads(const jl_mapfgpt_t* b) {
-    const int threads = build_threads(b->n_agents);
-    const bool few = b->n_envs <= 2 * device_cus() && b->n_agents > 2 * (threads / kWave);
+// for envs of at most 512 agents too where their LDS lets two such workgroups
+// share a CU and an env has more than a pair of egos for each wavefront: its
+// egos and changed fields then run on twice the wavefronts, which a batch of few
+// envs leaves idle otherwise.  While every env has a CU of its own that is
+// always faster (builds that keep their fields, 512 -> 1,024 threads: 1 env of
+// 64 agents 10.2 -> 8.8 us, 256 of 33 9.8 -> 9.1, of 128 17.8 -> 14.1).  Where
+// two share a CU it is slower for small envs, whose workgroups mostly start
+// and stage (400 of 48 10.9 -> 11.9 us, of 64 12.6 -> 12.7), and faster for
+// larger ones (of 88 15.7 -> 14.6, of 128 19.4 -> 17.8; 512 of 100 18.8 ->
+// 19.0), except that a build of raw rows, a training stage, mostly has envs
+// that start an episode, whose searches it shortens (512 of 40, 16 of them
+// starting: 64.6 -> 60.9 us; of 100 142 -> 132; without a start 11.3 -> 12.3).
+// With more envs than that, four workgroups of 512 threads per CU run in one
+// round where two of 1,024 would take two.
+int launch_threads(const jl_mapfgpt_t* b, bool rows) {
+    const int threads = build_threads(b->n_agents), cus = device_cus();
+    const bool few = b->n_agents > 2 * (threads / kWave) &&
+                     (b->n_envs <= cus || (b->n_envs <= 2 * cus && (rows || b->n_agents > 64)));
     return few && build_layout(b->n_agents, b->map_w, b->map_h, 1024 / kWave).total <= kLdsBytes / 2 ? 1024 : threads;
 }
 
 template <int H, bool kRows>
 int launch_single(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx, const int16_t* cy,
                   const int16_t* gx, const int16_t* gy, hipStream_t stream) {
-    const int threads = launch_threads(b);
+    const int threads = launch_threads(b, kRows);
     const size_t lds = build_layout(b->n_agents, b->map_w, H, threads / kWave).total;
     const dim3 grid(b->n_envs);
 #define JL_LAUNCH_BUILD(R, T)                                                                      \

@@ -48,3 +48,26 @@ def test_split_searches_run_at_once(W, H):
     assert got[0].groups <= cus() * (LDS // got[0].lds), got
     # and for at least 12 of a CU's 16 wavefronts (five-wavefront groups: 15)
     assert (LDS // got[0].lds) * got[0].threads >= 12 * 64, got
+
+
+# both sides of every line of the rule, and what small envs of a raw-row build take
+@pytest.mark.parametrize("E,A,rows,threads", [(1, 16, 0, 512), (1, 17, 0, 1024), (256, 33, 0, 1024), (257, 64, 0, 512),
+                                              (257, 65, 0, 1024), (257, 33, 1, 1024), (512, 65, 0, 1024),
+                                              (513, 65, 0, 512), (513, 65, 1, 512), (700, 513, 0, 1024)])
+def test_single_launch_workgroup_size(E, A, rows, threads):
+    """1,024 threads where an env has a CU of its own; where two envs share
+    one, only for envs large enough to gain from it, or raw rows."""
+    from iclr_2027_jointoom_amd import profile
+    from launches import launches
+
+    if cus() != 256:
+        pytest.skip("sizes of a card of 256 CUs")
+    b = profile(32, 32).MapfGPTObservationBuilder(torch.zeros((E, 32, 32), dtype=torch.int32, device="cuda"), A)
+    st = [torch.zeros((E, A), dtype=torch.int16, device="cuda")] * 4
+    raw = torch.zeros((E * A, 13), dtype=torch.int16, device="cuda")
+    call = (lambda: b.build_tokens(raw)) if rows else (lambda: b.build_tokens_from_state(*st))
+    call()
+    torch.cuda.synchronize()
+    got = [k for k in launches(call) if "build_kernel" in k.name]
+    assert len(got) == 1 and b.single_launch
+    assert (got[0].groups, got[0].threads) == (E, threads), got
