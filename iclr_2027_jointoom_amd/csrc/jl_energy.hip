@@ -17,6 +17,8 @@
 // 128 x 128 maps: 6.46 -> 0.22 ms (before: one wavefront per 64 jobs, one
 // after the other, with an LDS write per cell and level); 131,072 of 64 x 64:
 // 2.00 -> 0.40 ms (before the search by colour).
+#include <type_traits>
+
 #include "jl_bfs.h"
 #include "jl_common.h"
 
@@ -35,11 +37,34 @@ constexpr int energy_waves() {
 template <int H, int R, bool kSplit, int kWaves = energy_waves<H, R, kSplit>()>
 using EnergyLds = SearchLds<H, R, kSplit, false, kWaves>;
 
+// Planes of the highest level bits in LDS (flipped once in 64 and 128 levels),
+// where the registers have no room for them, of maps of at most kRows rows:
+// one wavefront's [plane][word][row].
+template <int N, int kRows>
+struct LdsPlanes {
+    uint32_t* words;
+    __device__ __forceinline__ uint32_t* word(int p, int i) const {
+        return words + (p * N + i) * kRows + (threadIdx.x & (kRows - 1));
+    }
+    __device__ __forceinline__ uint32_t value(int p, int i) const { return *word(p, i); }
+    __device__ __forceinline__ void flip(int p, bool first, const uint32_t (&a)[N]) const {
+        if ((threadIdx.x & (kWave - 1)) < kRows) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) *word(p, i) = first ? a[i] : *word(p, i) ^ a[i];
+        }
+    }
+};
+struct NoPlanes : NoTallPlanes {
+    __device__ __forceinline__ uint32_t value(int, int) const { return 0; }
+};
+
 // One field by the calling wavefront (kSplit: the workgroup, each wavefront on
 // its rows); every lane calls it with uniform arguments, the goal on the map.
-template <int H, int R, bool kSplit, typename Lds>
+template <int H, int R, bool kSplit, int kHigh = kEnergyHigh, typename Lds, typename Tall = NoPlanes>
 __device__ __forceinline__ void energy_field(const uint32_t* __restrict__ env_bits, int W, int gx, int gy,
-                                             uint8_t* __restrict__ out, int wave, int waves, Lds& s) {
+                                             uint8_t* __restrict__ out, int wave, int waves, Lds& s,
+                                             const Tall& tall = {}) {
+    static_assert(kHigh == kEnergyHigh || (kHigh == kEnergyHigh - 2 && !std::is_same_v<Tall, NoPlanes>), "every level bit");
     using S = SearchShape<H, R>;
     constexpr int HW = S::HW, N = S::N;
     // (taken afresh for every field: the addresses that follow from it would
@@ -47,9 +72,9 @@ __device__ __forceinline__ void energy_field(const uint32_t* __restrict__ env_bi
     int lane = threadIdx.x & (kWave - 1);
     asm volatile("" : "+v"(lane));
     const int x0 = (kSplit ? wave * S::kStep : 0) + lane * R;
-    SearchPlanes<H, R, kEnergyHigh> P;
+    SearchPlanes<H, R, kHigh> P;
     load_search_rows<H, R>(env_bits, W, x0, P.avail);
-    search_rows<H, R, kSplit, kEnergyHigh, kEnergyBatches, false>(P, gx, gy, x0, lane, wave, waves, s, NoTallPlanes{});
+    search_rows<H, R, kSplit, kHigh, kEnergyBatches, false>(P, gx, gy, x0, lane, wave, waves, s, tall);
     uint32_t vis[N];
     load_search_rows<H, R>(env_bits, W, x0, vis);
     const bool own = own_lane<H, R, kSplit>(lane, wave, waves);
@@ -61,6 +86,14 @@ __device__ __forceinline__ void energy_field(const uint32_t* __restrict__ env_bi
         // bits of 255 - d: each level bit inverted, none of an unreached cell
         const uint32_t e0 = v & (((x + gx + gy) & 1) ? 0xAAAAAAAAu : 0x55555555u);
         asm volatile("" ::: "memory");  // one word after the other (registers)
+        uint32_t p6, p7;  // level bits 6 and 7
+        if constexpr (kHigh == kEnergyHigh) {
+            p6 = P.high[2][i];
+            p7 = P.high[3][i];
+        } else {
+            p6 = P.tall > 0 ? tall.value(0, i) : 0u;
+            p7 = P.tall > 1 ? tall.value(1, i) : 0u;
+        }
         if (own && x < W) {
             uint4* row = reinterpret_cast<uint4*>(out + (size_t)x * H + k * 32);
 #pragma unroll 1
@@ -69,8 +102,7 @@ __device__ __forceinline__ void energy_field(const uint32_t* __restrict__ env_bi
 #pragma unroll
                 for (uint32_t q = 0; q < 2; ++q) {
                     const uint32_t lo = gather_bytes(e0, v & ~P.low[0][i], v & ~P.low[1][i], v & ~P.low[2][i], 2 * h + q);
-                    const uint32_t hi = gather_bytes(v & ~P.high[0][i], v & ~P.high[1][i], v & ~P.high[2][i],
-                                                     v & ~P.high[3][i], 2 * h + q);
+                    const uint32_t hi = gather_bytes(v & ~P.high[0][i], v & ~P.high[1][i], v & ~p6, v & ~p7, 2 * h + q);
                     b[q] = transpose8x8((uint64_t)hi << 32 | lo);
                 }
                 row[h] = make_uint4((uint32_t)b[0], (uint32_t)(b[0] >> 32), (uint32_t)b[1], (uint32_t)(b[1] >> 32));
@@ -193,6 +225,12 @@ __global__ __launch_bounds__(kRefreshThreads) void goal_changed_refresh_kernel(j
     __shared__ int64_t s_all[kRefreshWaves];
     __shared__ uint32_t s_scan[kRefreshWaves];
     __shared__ uint32_t s_goal[kRefreshThreads];  // (held in LDS: the search leaves no registers for it)
+    // 16 wavefronts have 128 registers each, which do not hold a search of
+    // rows of eight words: it keeps two level planes in LDS (10,000 agents on 16
+    // x 256 maps, no goal changed: 5.0 us; as two launches, 8.0)
+    constexpr int kWords = SearchShape<H, 1>::N, kMaxRows = kMarkedCells / H;
+    constexpr bool kLdsPlanes = kWords >= 8;
+    __shared__ uint32_t s_planes[kLdsPlanes ? kRefreshWaves : 1][kLdsPlanes ? 2 * kWords * kMaxRows : 1];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // uniform per wavefront
     const int A = s.n_agents, W = s.map_w;
@@ -272,8 +310,14 @@ __global__ __launch_bounds__(kRefreshThreads) void goal_changed_refresh_kernel(j
         const int x = (int)(goal & 0xFFFFu), y = (int)(goal >> 16);
         const int gi = c0 + wave * kWave + src;
         const int e = gi / A;
-        energy_field<H, 1, false>(s.grid_bits + (size_t)e * (cells / 32), W, x, y, energy + (size_t)gi * cells, wave,
-                                  kRefreshWaves, s_search);
+        const uint32_t* bits = s.grid_bits + (size_t)e * (cells / 32);
+        uint8_t* out = energy + (size_t)gi * cells;
+        if constexpr (kLdsPlanes) {
+            energy_field<H, 1, false, kEnergyHigh - 2>(bits, W, x, y, out, wave, kRefreshWaves, s_search,
+                                                       LdsPlanes<kWords, kMaxRows>{s_planes[wave]});
+        } else {
+            energy_field<H, 1, false>(bits, W, x, y, out, wave, kRefreshWaves, s_search);
+        }
     }
 }
 
@@ -390,14 +434,11 @@ extern "C" int jl_goal_changed_refresh(const jl_sim_t* s, uint8_t* energy, int64
     if (changed_states && (!s->cur_x || !s->cur_y || !s->actions)) return JL_ERR_ARG;
     const int64_t N = (int64_t)s->n_envs * s->n_agents;
     const int cells = s->map_w * s->map_h;
-    // (rows of 256 columns: 16 wavefronts of that search would not fit the
-    // registers)
-    if (N <= (int64_t)kRefreshThreads * kRefreshGroups && s->map_w <= kWave && cells <= 4096 && s->map_h < 256) {
+    if (N <= (int64_t)kRefreshThreads * kRefreshGroups && s->map_w <= kWave && cells <= 4096) {
         const unsigned grid = (unsigned)((N + kRefreshThreads - 1) / kRefreshThreads);
         JL_DISPATCH_H(s->map_h, {
-            if constexpr (H < 256)
-                hipLaunchKernelGGL(goal_changed_refresh_kernel<H>, dim3(grid), dim3(kRefreshThreads), 0,
-                                   (hipStream_t)stream, *s, energy, prefix, count, changed_states);
+            hipLaunchKernelGGL(goal_changed_refresh_kernel<H>, dim3(grid), dim3(kRefreshThreads), 0,
+                               (hipStream_t)stream, *s, energy, prefix, count, changed_states);
         });
         return launch_status();
     }

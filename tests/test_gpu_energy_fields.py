@@ -107,3 +107,32 @@ def test_many_fields_then_the_flagged_ones(oracle, W, H, E, A):
     e, a = np.nonzero(flags)
     assert int(sim.goal_changed_count.item()) == len(e)
     assert np.array_equal(packed[: len(e), :2], np.stack([e, a], 1)) and not packed[len(e):].any()
+
+
+@pytest.mark.parametrize("W,H", [(16, 256), (13, 256), (1, 256), (18, 224), (64, 64), (64, 32)])
+def test_refresh_of_changed_goals_in_one_launch(oracle, W, H):
+    """Maps of at most 4,096 cells and 64 rows: scan, packed rows and the
+    changed goals' fields (of distances past the cap) in a single launch."""
+    from iclr_2027_jointoom_amd import profile
+    from launches import launches
+
+    rng = np.random.default_rng(W * 3 + H)
+    grids, A = maps(W, H, W + H), 40
+    E = len(grids)
+    rows = state_rows(rng, grids, A)
+    goals = np.ascontiguousarray(rows[..., 4:6])
+    sim = profile(W, H).GridWorldSimulator(torch.from_numpy(grids.astype(np.int32)).cuda(), A, 0, E * W * H, 1,
+                                           "standard_mapf", 64)
+    sim.load_state(torch.from_numpy(goals).cuda(), torch.from_numpy(goals).cuda(),
+                   torch.zeros((E, A), dtype=torch.uint8, device="cuda"), torch.zeros(E, dtype=torch.int32, device="cuda"))
+    flags = (rng.random((E, A)) < 0.6).astype(np.uint8)
+    sim.current_step = 2
+    sim.goal_changed_flags.copy_(torch.from_numpy(flags).cuda())
+    sim.energy_maps.fill_(7)
+    sim.update_derived_state()
+    torch.cuda.synchronize()
+    flat = rows.reshape(-1, 8)
+    want = oracle.energy_maps(grids, flat.view(np.uint16), len(flat), A).reshape(E, A, -1)
+    got = sim.energy_maps.cpu().numpy().reshape(E, A, -1)
+    assert np.array_equal(got[flags == 1], want[flags == 1]) and (got[flags == 0] == 7).all()
+    assert [k.name for k in launches(sim.update_derived_state) if "refresh_kernel" not in k.name] == []
