@@ -134,15 +134,14 @@ __host__ __device__ inline NodeLayout node_layout(int A, int W, int H) {
 // agents, goal, ctg) of its cells into an LDS row that leaves as 16-byte
 // stores.
 //
-// A slice's rows may be shared by several workgroups (`share` of its agents
+// A slice's rows may be shared by `shares` workgroups (`share` of its agents
 // each, kNodeEgos where one takes them all): each stages the env and windows
 // of its own agents, the first one counts the slice's neighbours.
 template <int H>
-__global__ __launch_bounds__(kNodeThreads) void nodes_kernel(jl_magat_t m, int share) {
+__global__ __launch_bounds__(kNodeThreads) void nodes_kernel(jl_magat_t m, int share, int shares) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int A = m.n_agents, W = m.map_w, E = m.n_envs;
     const int parts = (A + kNodeEgos - 1) / kNodeEgos;
-    const int shares = kNodeEgos / share;
     const int slice = blockIdx.x / shares;
     const int env = slice / parts;
     const int part = slice - env * parts;
@@ -842,16 +841,19 @@ extern "C" int jl_magat_nodes(const jl_magat_t* m, jl_stream_t stream) {
     const NodeLayout L = node_layout(m->n_agents, m->map_w, m->map_h);
     const unsigned parts = (unsigned)((m->n_agents + kNodeEgos - 1) / kNodeEgos);
     // a slice's rows are shared out, down to one per wavefront, while the
-    // workgroups do not fill the CUs (4 envs of 48 agents: 18.2 -> 6.9 us).
+    // workgroups do not fill the CUs (one and several workgroups per slice, 64 x
+    // 64 maps: 4 envs of 48 agents 16.4 and 6.4 us, 250 of 64 21.8 and 15.1).
+    // Only agents that a slice has count: shares past them, every second
+    // workgroup, left half of the XCDs idle (148 envs of 16 agents on 256 x 256
+    // maps 12.5 us, 8.8 without them and 10.6 unshared).
+    const int egos = m->n_agents < kNodeEgos ? m->n_agents : kNodeEgos;
     int share = kNodeEgos;
-    while (share > kNodeThreads / kWave &&
-           (uint64_t)m->n_envs * parts * (kNodeEgos / share) < (uint64_t)device_cus())
-        share /= 2;
-    const unsigned shares = (unsigned)(kNodeEgos / share);
+    const auto shares = [&] { return (unsigned)((egos + share - 1) / share); };
+    while (share > kNodeThreads / kWave && (uint64_t)m->n_envs * parts * shares() < (uint64_t)device_cus()) share /= 2;
     JL_DISPATCH_H(m->map_h, {
         if (!lds_fits<&nodes_kernel<H>>(L.total)) return JL_ERR_AGENTS;
-        hipLaunchKernelGGL((nodes_kernel<H>), dim3((unsigned)m->n_envs * parts * shares), dim3(kNodeThreads),
-                           L.total, (hipStream_t)stream, *m, share);
+        hipLaunchKernelGGL((nodes_kernel<H>), dim3((unsigned)m->n_envs * parts * shares()), dim3(kNodeThreads),
+                           L.total, (hipStream_t)stream, *m, share, (int)shares());
     });
     return launch_status();
 }

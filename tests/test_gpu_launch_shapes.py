@@ -71,3 +71,18 @@ def test_single_launch_workgroup_size(E, A, rows, threads):
     got = [k for k in launches(call) if "build_kernel" in k.name]
     assert len(got) == 1 and b.single_launch
     assert (got[0].groups, got[0].threads) == (E, threads), got
+
+
+@pytest.mark.parametrize("E,A", [(1, 1), (148, 16), (200, 30), (239, 9), (4, 48), (250, 64), (300, 20)])
+def test_node_workgroups_all_have_rows(E, A):
+    """An env of at most 64 agents has no node workgroup without an agent
+    (every second one idle would leave half of the XCDs idle)."""
+    from iclr_2027_jointoom_amd import profile
+    from launches import launches
+
+    sim = profile(64, 64).GridWorldSimulator(torch.zeros((E, 64, 64), dtype=torch.int32, device="cuda"), A, 0,
+                                             E * 4096, 1, "standard_mapf", 64)
+    got = [k for k in launches(sim.build_magat_plus_nodes) if "nodes_kernel" in k.name]
+    assert len(got) == 1
+    # E workgroups of all A agents, or of a power of two of them, 4 to 32
+    assert got[0].groups in [E * -(-A // n) for n in (64, 32, 16, 8, 4)], got
