@@ -104,7 +104,8 @@ __device__ __forceinline__ void observe_agents(const jl_sim_t& s, const jl_mapfg
     const int pxl = s.cur_x[il], pyl = s.cur_y[il];
     const int32_t bestl = best[il];
     const int resetl = b.state_packed[(size_t)il * 8 + 7];
-    const uint32_t maskl = field_mask(b.cost_tiles, (uint32_t)il, W, H, A, tcells);
+    const uint32_t env_cell = marked_fields(W, H) ? kUnreachable
+                                                  : b.cost_tiles[env_plain_cell((uint32_t)il, A, tcells)];
     // window cells t0 = lane, t1 = lane + 64 (a cell when < 121); t = r*11 + c
     // is (cx + r - 5, cy + c - 5)
     const int t0 = lane, t1 = lane + kWave;
@@ -134,6 +135,8 @@ __device__ __forceinline__ void observe_agents(const jl_sim_t& s, const jl_mapfg
         w0[k] = ocp[c0[k] >> 5];
         w1[k] = ocp[c1[k] >> 5];
     }
+    // (after the windows' loads, which do not wait for it)
+    const uint32_t maskl = plain_field(b.cost_tiles, (uint32_t)il, env_cell, tcells) ? kPlainMask : kMarkedMask;
 #pragma unroll
     for (int k = 0; k < kObsPer; ++k) {
         if (k >= nvalid) break;  // wavefront-uniform
