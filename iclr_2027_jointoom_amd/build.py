@@ -2,7 +2,8 @@
 
 libjointloom.so is the product: the C ABI of include/jointloom.h.
 libjl_bench.so holds the HBM streaming probe that only bench.py (and its
-test) loads for the achievable-bandwidth figure; it is not part of the path.
+test) loads for the achievable-bandwidth figure, and a probe of the row
+search's counting that only its test loads; it is not part of the path.
 Each source compiles to its own object in parallel, then each library links.
 """
 from __future__ import annotations
@@ -17,7 +18,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 SOURCES = ["jl_sim.hip", "jl_mapfgpt.hip", "jl_energy.hip", "jl_magat.hip", "jl_records.hip",
            "jl_costtracer.hip"]
-BENCH_SOURCES = ["bench/jl_stream.hip"]
+BENCH_SOURCES = ["bench/jl_stream.hip", "bench/jl_search_count.hip"]
 OUTPUT = PKG_DIR / "libjointloom.so"
 BENCH_OUTPUT = PKG_DIR / "libjl_bench.so"
 

@@ -641,9 +641,10 @@ struct NoTallPlanes {
 // The search from (gx, gy) (inside the map; reached whether free or not) over
 // the free rows in P.avail.  kCap: levels from 16 * kCap on stay unreached
 // (0: no cap).  Returns, when kCount, the sum over levels of max(0, cells -
-// kMaxFrontier).  Every lane of the wavefront (kSplit: of the workgroup)
+// kLimit).  Every lane of the wavefront (kSplit: of the workgroup)
 // calls it with the same goal, and with the first of its map rows in x0.
-template <int H, int R, bool kSplit, int kHigh, int kCap, bool kCount, typename Lds, typename Tall>
+template <int H, int R, bool kSplit, int kHigh, int kCap, bool kCount, int kLimit = kMaxFrontier, typename Lds,
+          typename Tall>
 __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx, int gy, int x0, int lane, int wave, int waves,
                                            Lds& s, const Tall& tall) {
     using S = SearchShape<H, R>;
@@ -687,7 +688,7 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
         return c;
     };
     int slot = 0, cells = kCount ? reached_cells() : 0;
-    bool big = false;  // kCount: 8 levels of the batch reached more than kMaxFrontier cells
+    bool big = false;  // kCount: 8 levels of the batch reached more than kLimit cells
     // After kSplitLevels levels: whether any cell is left to expand (news:
     // this lane's last level reached one); sets big.  kSplit: the overlap is
     // taken from its owners.
@@ -700,8 +701,8 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
             cells = now;
         }
         if constexpr (!kSplit) {
-            // more than kMaxFrontier cells need a lane with more than its share
-            if (kCount && __any(reached > kMaxFrontier / kWave)) big |= wave_sum(reached) > kMaxFrontier;
+            // more than kLimit cells need a lane with more than its share
+            if (kCount && __any(reached > kLimit / kWave)) big |= wave_sum(reached) > kLimit;
             return __any(left) != 0;
         } else {
             const bool lo = lane >= G && lane < 2 * G, hi = lane >= kWave - 2 * G && lane < kWave - G;
@@ -729,8 +730,8 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
             slot ^= 1;
             // (the wavefronts' counts are added up only where one of them
             // has more than its share)
-            if (kCount && __any((int)(all >> 1) * waves > kMaxFrontier))
-                big |= wave_sum(lane < waves ? (int)(all >> 1) : 0) > kMaxFrontier;
+            if (kCount && __any((int)(all >> 1) * waves > kLimit))
+                big |= wave_sum(lane < waves ? (int)(all >> 1) : 0) > kLimit;
             return __any(all & 1u) != 0;
         }
     };
@@ -827,15 +828,15 @@ __device__ __forceinline__ int search_rows(SearchPlanes<H, R, kHigh>& P, int gx,
                 c = wave_sum(mine ? c : 0);
                 if (kSplit) {
                     if (lane == 0) atomicAdd(&s.count[v], (uint32_t)c);
-                } else if (c > kMaxFrontier) {
-                    overflow += c - kMaxFrontier;
+                } else if (c > kLimit) {
+                    overflow += c - kLimit;
                 }
             }
             if (kSplit) {
                 lds_barrier();
                 for (int v = 0; v < 16; ++v) {
                     const int c = __builtin_amdgcn_readfirstlane((int)s.count[v]);
-                    if (c > kMaxFrontier) overflow += c - kMaxFrontier;
+                    if (c > kLimit) overflow += c - kLimit;
                 }
                 lds_barrier();
             }
