@@ -109,14 +109,11 @@ __device__ __forceinline__ void load_free_rows(const uint32_t* __restrict__ env_
     }
 }
 
-// Runs the BFS from (gx, gy) (which must be inside the map; it is visited
-// even when it is an obstacle, as the energy BFS does) and writes
-// dist[x*H+y] = level for every reached cell except the start, for levels
-// 1..cap.  dist must already hold the "unreached" value and the start cell
-// its 0.
-template <int H, int R, typename T>
-__device__ void wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int gy, int cap,
-                        T* dist) {
+// Runs the BFS from the free cell (gx, gy) and writes dist[x*H+y] = level for
+// every reached cell except the start.  dist must already hold the
+// "unreached" value and the start cell its 0.
+template <int H, int R>
+__device__ void wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int gy, uint16_t* dist) {
     constexpr int HW = RowWords<H>::HW;
     const int lane = threadIdx.x & (kWave - 1);
     uint64_t front[R][HW];
@@ -144,7 +141,7 @@ __device__ void wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int g
             }
         }
     }
-    for (int level = 1; level <= cap; ++level) {
+    for (int level = 1;; ++level) {
         uint64_t nf[R][HW];
         bool any_new = false;
 #pragma unroll
@@ -182,12 +179,12 @@ __device__ void wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int g
                 uint64_t m = nf[r][k];
                 // two new cells per pass, the lowest and the highest (the same
                 // cell twice when one is left)
-                T* row_dist = dist + x * H + k * 64;
+                uint16_t* row_dist = dist + x * H + k * 64;
                 while (m) {
                     const int lo = __ffsll((unsigned long long)m) - 1;
                     const int hi = 63 - __clzll((long long)m);
-                    row_dist[lo] = (T)level;
-                    row_dist[hi] = (T)level;
+                    row_dist[lo] = (uint16_t)level;
+                    row_dist[hi] = (uint16_t)level;
                     m &= ~((1ull << lo) | (1ull << hi));
                 }
             }
@@ -195,9 +192,8 @@ __device__ void wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int g
     }
 }
 
-// wave_bfs for one row per lane (R = 1) without a level cap, in batches of 16
-// levels: the levels of a batch
-// are unrolled into straight-line code (expansion, then the new cells ORed
+// wave_bfs for one row per lane (R = 1), in batches of 16 levels: the levels
+// of a batch are unrolled into straight-line code (expansion, then the new cells ORed
 // into the batch mask and into the planes of the level's 4 low bits, chosen
 // at compile time), and only after the batch are its cells' distances
 // L0 + (plane bits) written, one pass over the batch mask.  The search stops
@@ -205,8 +201,8 @@ __device__ void wave_bfs(const uint64_t (&fr)[R][RowWords<H>::HW], int gx, int g
 // last reach nothing, so the field is wave_bfs's).  The single wavefront's
 // search is a chain of dependent instructions; the batch keeps the writes
 // off that chain and lets the plane and mask updates fill its gaps.
-template <int H, typename T>
-__device__ void wave_bfs_batched(const uint64_t (&fr)[RowWords<H>::HW], int gx, int gy, T* dist) {
+template <int H>
+__device__ void wave_bfs_batched(const uint64_t (&fr)[RowWords<H>::HW], int gx, int gy, uint16_t* dist) {
     constexpr int HW = RowWords<H>::HW;
     constexpr int kBatch = 16;
     const int lane = threadIdx.x & (kWave - 1);
@@ -220,7 +216,7 @@ __device__ void wave_bfs_batched(const uint64_t (&fr)[RowWords<H>::HW], int gx, 
             avail[k] &= ~front[k];
         }
     }
-    T* row_dist = dist + lane * H;
+    uint16_t* row_dist = dist + lane * H;
     for (int L0 = 1;; L0 += kBatch) {
         uint64_t bm[HW], p0[HW], p1[HW], p2[HW], p3[HW];
 #pragma unroll
@@ -255,7 +251,7 @@ __device__ void wave_bfs_batched(const uint64_t (&fr)[RowWords<H>::HW], int gx, 
                 const int c = __ffsll((unsigned long long)m) - 1;
                 const uint32_t j = (uint32_t)((p0[k] >> c) & 1u) | (uint32_t)((p1[k] >> c) & 1u) << 1 |
                                    (uint32_t)((p2[k] >> c) & 1u) << 2 | (uint32_t)((p3[k] >> c) & 1u) << 3;
-                row_dist[k * 64 + c] = (T)(L0 + (int)j);
+                row_dist[k * 64 + c] = (uint16_t)(L0 + (int)j);
                 m &= m - 1;
             }
         }
@@ -266,8 +262,9 @@ __device__ void wave_bfs_batched(const uint64_t (&fr)[RowWords<H>::HW], int gx, 
     }
 }
 
-// Planes of the levels of a search on a map of at most 4,096 cells (levels
-// stay below 4,096): four low planes in registers, eight high ones in LDS.
+// Level bits of a search on a map of at most 4,096 cells (levels stay below
+// 4,096): bit 0 is the cell's colour, bits 1-3 are planes in registers, the
+// eight high ones planes in LDS.
 constexpr int kFieldPlanes = 12;
 constexpr int kHighPlanes = kFieldPlanes - 4;
 // LDS of one wavefront's high planes: [plane][lane] 64-bit words.
@@ -467,13 +464,6 @@ __host__ __device__ constexpr int split_waves(int W) {
     const int rows = (W + 7) / 8 * 8;
     return rows <= kWave * R ? 1
                              : (rows - kWave * R + SearchShape<H, R>::kStep - 1) / SearchShape<H, R>::kStep + 1;
-}
-
-// Bits of the levels of a search over `cells` cells (levels stay below it).
-__host__ __device__ constexpr int level_bits(int cells) {
-    int b = 0;
-    while ((1 << b) < cells) ++b;
-    return b;
 }
 
 // LDS of one wavefront of a search.

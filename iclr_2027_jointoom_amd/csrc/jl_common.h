@@ -201,13 +201,6 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// 64-bit cross-lane read (ds_bpermute); lanes outside [0,64) wrap.
-__device__ __forceinline__ uint64_t shfl64(uint64_t v, int src_lane) {
-    const int lo = __shfl((int)(uint32_t)v, src_lane, kWave);
-    const int hi = __shfl((int)(uint32_t)(v >> 32), src_lane, kWave);
-    return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
-}
-
 __device__ __forceinline__ int coord_token(int v) {
     v = v < -kCostLimit ? -kCostLimit : v;
     v = v > kCostLimit ? kCostLimit : v;

@@ -366,9 +366,9 @@ __device__ uint32_t refresh_field(const jl_mapfgpt_t& b, size_t agent_index, uin
         if (lane == 0) s_dist[gx * H + gy] = 0;
         wave_sync();
         if constexpr (R == 1) {
-            wave_bfs_batched<H, uint16_t>(fr[0], gx, gy, s_dist);
+            wave_bfs_batched<H>(fr[0], gx, gy, s_dist);
         } else {
-            wave_bfs<H, R, uint16_t>(fr, gx, gy, 0x7FFFFFFF, s_dist);
+            wave_bfs<H, R>(fr, gx, gy, s_dist);
         }
     }
     wave_sync();
@@ -601,8 +601,7 @@ __device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, si
 // field, one whose reset flag is set is listed in LDS.  Then the listed
 // fields are searched: by one wavefront each where a wavefront holds the
 // whole map (W <= 64 R), or (kSplit) by the whole workgroup one after the
-// other.  A build without a
-// changed goal is the unpack alone.
+// other.  A build without a changed goal is the unpack alone.
 //
 // The grid is the workgroups resident at once (field_waves_per_simd and the
 // LDS of the wavefronts that the map needs, launch_fields), or one per
@@ -696,9 +695,10 @@ __host__ __device__ inline size_t marked_wave_lds(int W, int H) {
 
 // ---------------------------------------------------------------------------
 // Pass 1 for maps of at most kMarkedCells cells (8 KB fields) when the
-// single-launch build does not apply: one lane per agent and 4 wavefronts per workgroup, each wavefront refreshing the fields
-// of its own agents whose goal changed in its LDS field.  The tiled copies
-// it writes carry the greedy marks (jl_common.h, marked_fields).
+// single-launch build does not apply: one lane per agent and 4 wavefronts per
+// workgroup, each wavefront refreshing the fields of its own agents whose goal
+// changed in its LDS field.  The tiled copies it writes carry the greedy marks
+// (jl_common.h, marked_fields).
 // ---------------------------------------------------------------------------
 template <int H, int R, bool kRows, int kWaves>
 __global__ __launch_bounds__(kWave* kWaves) void unpack_bfs_kernel(

@@ -267,7 +267,7 @@ int jl_mapfgpt_build_state(const jl_mapfgpt_t* b, const int16_t* cur_x,
  * 4096 cells with rows of at most 64 columns (map_h <= 64), an env of at
  * most 1024 agents, build_scratch set): unpack,
  * field refreshes and tokens of an env in one workgroup, also when captured
- * into a graph; 0 when it runs as two or three launches.  No
+ * into a graph; 0 when it runs as two launches.  No
  * counterpart in the reference (a profiling query: the token_events pair
  * then brackets the whole build). */
 int jl_mapfgpt_single_launch(const jl_mapfgpt_t* b);
