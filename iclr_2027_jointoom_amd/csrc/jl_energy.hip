@@ -14,9 +14,10 @@
 // changed goals: goal_changed_refresh_kernel).
 //
 // Bound by VALU issue when every field is new.  16,000 fields of i.i.d.
-// 128 x 128 maps: 6.46 -> 0.22 ms (before: one wavefront per 64 jobs, one
-// after the other, with an LDS write per cell and level); 131,072 of 64 x 64:
-// 2.00 -> 0.40 ms (before the search by colour).
+// 128 x 128 maps: 6.46 -> 0.19 ms (before: one wavefront per 64 jobs, one
+// after the other, with an LDS write per cell and level; now 6,497 VALU
+// instructions each, issue 1.0 of the time); 131,072 of 64 x 64, a third of
+// the cells obstacles: 2.06 -> 0.25 ms.
 #include <type_traits>
 
 #include "jl_bfs.h"
@@ -344,7 +345,12 @@ EnergyGrid energy_grid(int jobs, int W, bool every) {
 
 // f.template operator()<R, kSplit>() with the lane layout of a W x H map: a
 // wavefront on its own where its lanes' registers hold the rows (at most 8
-// words each), else the map split over a workgroup.
+// words each, 130 registers), else the map split over a workgroup.  A first MAGAT
+// stage of 64 envs of 128 agents, us, with this line at 4, 8 and 16 words (250
+// registers, none spilled): 128 x 96 179, 118, 118; 256 x 64 183, 124, 124; 100 x
+// 160 195, 194, 186; 160 x 128 205, 249, 231; 128 x 192 326, 326, 195; 256 x 96
+// 351, 380, 247; 256 x 128 351, 379, 243; 128 x 256 437, 437, 252.  So 8 against
+// 4 holds where a wavefront then is alone, and 16 would gain on the larger maps.
 template <int H, typename F>
 int with_energy_layout(int W, F f) {
     constexpr int kAlone = SearchShape<H, 4>::N <= 8 ? 4 : (SearchShape<H, 2>::N <= 8 ? 2 : 1);

@@ -607,13 +607,13 @@ __device__ __forceinline__ uint32_t refresh_field_rows(const jl_mapfgpt_t& b, si
 // LDS of the wavefronts that the map needs, launch_fields), or one per
 // wavefront's worth of agents, so that a batch of new fields covers the chip:
 // ranges rounded to whole passes of the workgroup's threads left 8,192
-// new fields to 64 (128 x 128) and 32 (256 x 256) workgroups.  Bound by VALU
-// issue when every field is new.  8,192 new fields of i.i.d. 128 x 128 maps
-// (issue-bound): 15.8 ms with a workgroup of two wavefronts, a barrier and a
-// 16-plane update per level -> 0.21 ms; of 256 x 256 warehouses (about 80 k
-// VALU wavefront instructions each, 1.1 ms of issue): 79.8 -> 1.8 ms.  Four
-// times as many groups in smaller ranges: 5 % and 3 % less, but a step that
-// keeps its fields took longer.  With the LDS of five wavefronts whatever the
+// new fields to 64 (128 x 128) and 32 (256 x 256) workgroups.  8,192 new
+// fields of i.i.d. 128 x 128 maps: 15.8 ms with a workgroup of two wavefronts,
+// a barrier and a 16-plane update per level -> 0.18 ms (8,226 VALU
+// instructions each, VALU issue 0.71 of the time); of 256 x 256 warehouses: 79.8
+// -> 1.8 ms (66,751 each, issue 0.51, the other half waits at the exchanges).
+// Four times as many groups in smaller ranges: 5 % and 3 % less, but a step
+// that keeps its fields took longer.  With the LDS of five wavefronts whatever the
 // map needs (three workgroups per CU instead of eight, five or four): 8,192 new
 // fields of 96 x 256 maps 765 us, 128 x 256 960, 200 x 256 1,200, 100 x 160
 // 359, against 432, 785, 985 and 258.  Without a changed goal (131,072 agents,
@@ -2089,7 +2089,14 @@ int launch_pass1(const jl_mapfgpt_t* b, const int16_t* rows, const int16_t* cx, 
         return launch_status();
     }
     // a wavefront searches alone where a map's rows fit its lanes' registers
-    // (at most 8 words per lane), else the map's rows are split
+    // at three wavefronts per SIMD (at most 8 words per lane), else the map's
+    // rows are split.  8,192 new fields, us, with this line at 4, 8 and 16 words
+    // (16: two wavefronts per SIMD and 20-32 registers spilled): 128 x 96 287, 152,
+    // 147; 128 x 128 313, 181, 179; 256 x 64 339, 275, 233; 100 x 160 259, 259,
+    // 235; 160 x 128 343, 354, 408; 256 x 128 838, 710, 701 (16,384 fields:
+    // 1,635, 1,303, 1,355); 128 x 192 521, 521, 325; 256 x 96 770, 649, 479; 128 x
+    // 256 788, 788, 501.  So 8 against 4 is clear, and maps of 16 words would gain
+    // from going alone if their planes found room without spilling.
     constexpr int kAlone = SearchShape<H, 4>::N <= 8 ? 4 : (SearchShape<H, 2>::N <= 8 ? 2 : 1);
     if constexpr (kWave * R * H <= kMarkedCells) return JL_ERR_PROFILE;  // always marked
     else if constexpr (R <= kAlone) return launch_fields<H, R, false, kRows>(b, rows, cx, cy, gx, gy, stream);
